@@ -14,6 +14,7 @@ the Python functions of corrfunc_amd.theory and corrfunc_amd.mocks on the caller
 """
 import ctypes
 import math
+import os
 
 import numpy as np
 import torch
@@ -222,7 +223,6 @@ class _BinFile:
         self.path = _abi.write_bin_file(edges)[0]
 
     def __del__(self):
-        import os
         try:
             os.remove(self.path)
         except Exception:
