@@ -24,7 +24,7 @@ struct BgOpts {
     int custom;         // custom refine factors: no 0.05-wrap rule and no boost
     int max_cells;      // options->max_cells_per_dim
     int min_sep_opt;
-    int64_t ncells_cap; // cells (and 16 z-slabs each) the catalog's buffers hold
+    int64_t ncells_cap; // cells the catalog's buffers hold
 };
 
 // Per-catalog plan written by k_bg_grid and read by the later steps.
@@ -146,29 +146,28 @@ __global__ void k_bg_grid(int k, BgOpts o, const double* __restrict__ ext, int64
 template <typename T>
 __global__ void k_bg_bucket_count(int64_t n, const T* __restrict__ X, const T* __restrict__ Y,
                                   const T* __restrict__ Z, const BgCat* __restrict__ cat, int* __restrict__ bucket,
-                                  int* __restrict__ counts, unsigned long long* __restrict__ oob)
+                                  int* __restrict__ rank, int* __restrict__ counts,
+                                  unsigned long long* __restrict__ oob)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) bucket_count_one(i, X, Y, Z, cat->g, bucket, counts, oob);
+    if (i < n) bucket_count_one(i, X, Y, Z, cat->g, bucket, rank, counts, oob);
 }
 
+// The cells' sort and boxes (k_build_small, k_build_big) with the grid the
+// device chose; B holds the catalog's buffers.
 template <typename T>
-__global__ void k_bg_scatter(int64_t n, const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-                             const T* __restrict__ W, const BgCat* __restrict__ cat, const int* __restrict__ bucket,
-                             const int* __restrict__ bstart, int* __restrict__ fill, double* __restrict__ x,
-                             double* __restrict__ y, double* __restrict__ z, double* __restrict__ w,
-                             double4* __restrict__ d4, uint2* __restrict__ q)
+__global__ __launch_bounds__(256) void k_bg_build_small(const T* X, const T* Y, const T* Z, const T* W,
+                                                        const BgCat* cat, DevLattice B, const int* idx, int* keys,
+                                                        int* big)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) scatter_one(i, X, Y, Z, W, cat->g, bucket, bstart, fill, x, y, z, w, d4, q);
+    build_small(cat->ncells, X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, big);
 }
-
-__global__ void k_bg_cell_bounds(const BgCat* __restrict__ cat, const int* __restrict__ bstart,
-                                 const double* __restrict__ x, const double* __restrict__ y,
-                                 const double* __restrict__ z, double* __restrict__ bounds)
+template <typename T>
+__global__ __launch_bounds__(kBigThreads) void k_bg_build_big(const T* X, const T* Y, const T* Z, const T* W,
+                                                              const BgCat* cat, DevLattice B, const int* idx,
+                                                              int* keys, const int* big)
 {
-    const int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-    if (c < cat->ncells) cell_bounds_one(c, bstart, x, y, z, bounds);  // uniform per wave
+    build_big(X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, big);
 }
 
 // Candidates (cell, neighbour) over the captured capacity `cap`; those beyond

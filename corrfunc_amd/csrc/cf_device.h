@@ -19,8 +19,14 @@ enum R2Form {
     RP_FMA = 11           // fma(dy,dy,dx*dx)                 AVX512F rp_pi / wp, AVX2 wp
 };
 
-// Number of z-slabs each cell is bucketed into by the gridding sort.
-constexpr int kSlabs = 16;
+// Particles of a cell are ordered along a Hilbert curve and carry one bounding
+// box per kGroup consecutive ones. The groups of cell c, whose particles start
+// at s, are numbered group_index(s, c) + 0, 1, ...: consecutive within a cell
+// and disjoint between cells without a scan of their counts (a cell of m
+// particles needs ceil(m / kGroup) <= floor((s + m) / kGroup) - floor(s / kGroup) + 1
+// numbers); n / kGroup + ncells + 1 boxes hold them all.
+constexpr int kGroup = 16;
+__host__ __device__ inline int64_t group_index(int s, int64_t c) { return s / kGroup + c; }
 
 // Quantized positions: |q| <= kQMax, so differences fit int16 and a sum of three
 // squared differences fits uint32; kQPad entries pad the array for block loads.
@@ -39,7 +45,7 @@ struct CellPairRec {
 };
 static_assert(sizeof(CellPairRec) == 64, "CellPairRec must be 64 bytes");
 
-// A gridded particle set resident in HBM, sorted by (cell, z-slab).
+// A gridded particle set resident in HBM, sorted by (cell, Hilbert order in the cell).
 struct DevLattice {
     int nx, ny, nz;
     int64_t ncells;
@@ -47,8 +53,7 @@ struct DevLattice {
     double xmin, ymin, zmin;
     double xbs, ybs, zbs;      // cell sizes
     double xinv, yinv, zinv;   // 1/cell size (0 if the size is 0)
-    double *x, *y, *z, *w;     // FP64 positions / weight, cell order
-    double4 *d4;               // the same as one 32-byte record (x, y, z, w) per particle
+    double4 *d4;               // one FP64 record (x, y, z, weight) per particle, cell order
     // Cell-local quantized positions for the integer pair filter: per particle
     // (qx & 0xffff) | (qy << 16) and qz, q = rint((x - ox) * qinv), ox = xmin + ix*xbs,
     // followed by kQPad padding entries.
@@ -58,7 +63,8 @@ struct DevLattice {
     int qlo_neg;
     int qz;                    // projected modes: pass iff |dqz| < qz
     int qpad_;
-    int *bstart;               // [ncells*kSlabs + 1] bucket starts
+    int *bstart;               // [ncells + 1] cell starts
+    double *gbox;              // [(n/kGroup + ncells + 1)*6] the groups' boxes, x lo,hi, y lo,hi, z lo,hi
     double *bounds;            // [ncells*6] x lo,hi, y lo,hi, z lo,hi
 };
 
@@ -80,19 +86,18 @@ struct PairParams {
     double max_all_dz_same;  // same-cell z window (DD/xi/s_mu)
     double xwrap, ywrap, zwrap;
     double near_r2, near_dz; // edge windows below which pruning replay is skipped
-    double zreach;           // z reach used for the slab window
-    double slab_margin;
+    double zreach;           // largest |dz| of a counted pair
+    double box_margin;       // slack of the group boxes' z test
     // bin lookup: slot count of edges below the 1/16-octave bucket of (float)r^2
     int lut_base;            // bucket index of lut[0]
     int lut_n;               // entries
     int lut_single;          // 1: no bucket holds more than one edge, so one compare finishes the lookup
-    int dense_mode;          // 0: by work-item flag, 1: always dense, 2: never dense
+    int dense_mode;          // 0: by group, 1: always dense, 2: never dense
     int hist_copies;         // LDS histogram replication R (power of 2): lane l adds to copy l % R
     int dense_stride;        // 1: dense work items take strided primaries
-    float dense_frac;        // a cell pair whose estimated in-range fraction reaches this takes the dense path
+    float dense_frac;        // a group whose estimated in-range fraction reaches this takes the dense path
     int fetch;               // work items per queue atomic outside the single-fetch ranges
     int prim_cache;          // 1: the sparse path keeps the wave's primaries in LDS for its drains
-    int max_window;          // longest secondary window scanned with one queue base (2^25, a multiple of 4)
     int qblock_log2;         // work items go to sub-queues in blocks of 2^qblock_log2 consecutive items
 };
 

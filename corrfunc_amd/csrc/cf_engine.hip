@@ -446,54 +446,66 @@ static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n,
     L.xmin = g.xmin; L.ymin = g.ymin; L.zmin = g.zmin;
     L.xbs = g.xbs; L.ybs = g.ybs; L.zbs = g.zbs;
     L.xinv = g.xinv; L.yinv = g.yinv; L.zinv = g.zinv;
-    const int64_t nb = L.ncells * kSlabs;
+    const int64_t nb = L.ncells;
     if (nb >= (int64_t)INT32_MAX || n >= (int64_t)INT32_MAX) {
         fprintf(stderr, "Error: grid of %lld cells or %lld particles exceeds the engine's 32-bit indexing\n",
                 (long long)L.ncells, (long long)n);
         return EXIT_FAILURE;
     }
+    const int64_t nbig = n / kSmallCell;  // at most this many cells hold more than kSmallCell particles
     int* counts = (int*)E.arena.get(tag + "_cnt", sizeof(int) * (nb + 1));
-    int* fill = (int*)E.arena.get(tag + "_fill", sizeof(int) * (nb + 1));
     int* bucket = (int*)E.arena.get(tag + "_bucket", sizeof(int) * (n + 1));
+    int* rank = (int*)E.arena.get(tag + "_rank", sizeof(int) * (n + 1));
+    int* idx = (int*)E.arena.get(tag + "_idx", sizeof(int) * (n + 1));
+    int* big = (int*)E.arena.get(tag + "_big", sizeof(int) * (nbig + 1));
     L.bstart = (int*)E.arena.get(tag + "_bstart", sizeof(int) * (nb + 1));
-    L.x = (double*)E.arena.get(tag + "_x", sizeof(double) * n);
-    L.y = (double*)E.arena.get(tag + "_y", sizeof(double) * n);
-    L.z = (double*)E.arena.get(tag + "_z", sizeof(double) * n);
-    L.w = W ? (double*)E.arena.get(tag + "_w", sizeof(double) * n) : nullptr;
     L.d4 = (double4*)E.arena.get(tag + "_d4", sizeof(double4) * (n + kQPad));
     // quantum: kQMax quanta cover the largest cell side plus the pair reach, so
     // every position within reach of a cell has an unclamped quantized offset
     L.qinv = (double)kQMax / (fmax(g.xbs, fmax(g.ybs, g.zbs)) + g.qreach);
     L.q = (uint2*)E.arena.get(tag + "_q", sizeof(uint2) * (n + kQPad));
     L.bounds = (double*)E.arena.get(tag + "_bounds", sizeof(double) * 6 * L.ncells);
+    L.gbox = (double*)E.arena.get(tag + "_gbox", sizeof(double) * 6 * (n / kGroup + L.ncells + 1));
     fill_i32(counts, nb + 1, 0);
-    fill_i32(fill, nb + 1, 0);
+    fill_i32(big, 1, 0);
     GridArgs ga{g.xmin, g.ymin, g.zmin, g.xinv, g.yinv, g.zinv, g.xbs, g.ybs, g.zbs, g.nx, g.ny, g.nz, L.qinv};
     const unsigned blocks = (unsigned)((n + 255) / 256);
     if (n > 0) {
         if (esize == 4)
             k_bucket_count<float><<<blocks, 256, 0, E.stream>>>(n, (const float*)X, (const float*)Y, (const float*)Z,
-                                                                 ga, bucket, counts, oob);
+                                                                 ga, bucket, rank, counts, oob);
         else
             k_bucket_count<double><<<blocks, 256, 0, E.stream>>>(n, (const double*)X, (const double*)Y,
-                                                                  (const double*)Z, ga, bucket, counts, oob);
+                                                                  (const double*)Z, ga, bucket, rank, counts, oob);
         CF_CHECK(hipGetLastError());
     }
     device_scan(counts, L.bstart, nb, tag + "_scan");
     if (n > 0) {
-        if (esize == 4)
-            k_scatter<float><<<blocks, 256, 0, E.stream>>>(n, (const float*)X, (const float*)Y, (const float*)Z,
-                                                            (const float*)W, ga, bucket, L.bstart, fill, L.x, L.y,
-                                                            L.z, L.w, L.d4, L.q);
-        else
-            k_scatter<double><<<blocks, 256, 0, E.stream>>>(n, (const double*)X, (const double*)Y, (const double*)Z,
-                                                             (const double*)W, ga, bucket, L.bstart, fill, L.x,
-                                                             L.y, L.z, L.w, L.d4, L.q);
+        k_index_scatter<<<blocks, 256, 0, E.stream>>>(n, bucket, rank, L.bstart, idx);
         CF_CHECK(hipGetLastError());
     }
-    k_cell_bounds<<<(unsigned)((L.ncells + 3) / 4), 256, 0, E.stream>>>(L.ncells, L.bstart, L.x, L.y, L.z,
-                                                                           L.bounds);
+    // (the cells' sort keys take the place of the ranks)
+    const unsigned sb = (unsigned)((L.ncells + 3) / 4), bb = (unsigned)std::min<int64_t>(nbig, 2 * E.ncu);
+    if (esize == 4)
+        k_build_small<float><<<sb, 256, 0, E.stream>>>(L.ncells, (const float*)X, (const float*)Y, (const float*)Z,
+                                                        (const float*)W, ga, L.bstart, idx, rank, L.d4, L.q,
+                                                        L.bounds, L.gbox, big);
+    else
+        k_build_small<double><<<sb, 256, 0, E.stream>>>(L.ncells, (const double*)X, (const double*)Y,
+                                                         (const double*)Z, (const double*)W, ga, L.bstart, idx,
+                                                         rank, L.d4, L.q, L.bounds, L.gbox, big);
     CF_CHECK(hipGetLastError());
+    if (bb > 0) {
+        if (esize == 4)
+            k_build_big<float><<<bb, kBigThreads, 0, E.stream>>>((const float*)X, (const float*)Y, (const float*)Z,
+                                                                  (const float*)W, ga, L.bstart, idx, rank, L.d4,
+                                                                  L.q, L.bounds, L.gbox, big);
+        else
+            k_build_big<double><<<bb, kBigThreads, 0, E.stream>>>((const double*)X, (const double*)Y,
+                                                                   (const double*)Z, (const double*)W, ga, L.bstart,
+                                                                   idx, rank, L.d4, L.q, L.bounds, L.gbox, big);
+        CF_CHECK(hipGetLastError());
+    }
     return EXIT_SUCCESS;
 }
 
@@ -727,7 +739,7 @@ static int choose_grid(int mode, int64_t N1, double rmax, double pimax, double b
 }
 
 // Launch parameters of the pair kernels: rounding order, cut values, edge
-// windows, slab window and the bin lookup table (the integer filter's
+// windows, z reach and the bin lookup table (the integer filter's
 // thresholds depend on the secondary set's quantum: set_quant_filter).
 static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, const std::vector<double>& rupp_sqr,
                          int sorted, double rmax, double pimax, double inv_d2, double sqr_mu_max, int need_avg,
@@ -765,7 +777,7 @@ static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, con
     P.near_r2 = 1e-9 * P.sqr_rmax + 1e-9 * rmax * coord_scale;
     P.near_dz = 1e-9 * pimax + 1e-9 * coord_scale;
     P.zreach = (is2d || mode == MODE_SMU) ? pimax : sqrt(P.sqr_rmax);
-    P.slab_margin = 1e-7 * (coord_scale + cs);
+    P.box_margin = 1e-7 * (coord_scale + cs);
 
     // ---- bin lookup table: for each 1/16-octave bucket of (float)r^2, the number
     // of edges strictly below the bucket (a lower bound of the bin index)
@@ -832,10 +844,6 @@ static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, con
         // (workload 5) 2.71 s at 0.35, 2.60 s at 0.2-0.25, 3.18 s at 0; DDrppi
         // and DD within 2 % from 0.2 to 0.5
         P.dense_frac = df ? (float)atof(df) : 0.25f;
-        // sub-window length of the sparse scan (tests shorten it to exercise the
-        // window changes; a multiple of 4 below 2^26)
-        const char* mw = getenv("CORRFUNC_AMD_MAX_WINDOW");
-        P.max_window = mw ? std::max(4, std::min(1 << 25, atoi(mw))) & ~3 : 1 << 25;
         const char* qb = getenv("CORRFUNC_AMD_QBLOCK_LOG2");
         // blocks of 32 items per sub-queue (measured, bench.py --sweep
         // CORRFUNC_AMD_QBLOCK_LOG2=0..8): DDsmu cross -1.8 %, DDrppi -1.5 %, DD and xi
@@ -1555,7 +1563,7 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
         build_params(mode, resolve_isa(o->instruction_set), nbin, n2, (int)nslots, rupp_sqr, sorted, rmax, pimax,
                      inv_d2, sqr_mu_max, o->need_avg_sep, need_w, c.autocorr, wrap, coord_scale, cs, rmaxr, P, lut);
         if (onsky) {
-            // 3-D limit for the pruning, the filter and the slab window; rp^2 limit
+            // 3-D limit for the pruning, the filter and the z reach; rp^2 limit
             // for the (rp, pi) bins (countpairs_rp_pi_mocks_impl.c.src:303-306)
             P.sqr_rpmax = rupp_sqr[nbin - 1];
             P.sqr_rmax = mode == MODE_RPPI_MOCKS ? rmax * rmax + pimax * pimax : rupp_sqr[nbin - 1];
@@ -1619,7 +1627,7 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     if (need_w) {
         double* ws = (double*)E.arena.get("wsums", sizeof(double) * 2);
         fill_u64(ws, 2);
-        if (c.N1 > 0) k_weight_sums<<<256, 256, 0, E.stream>>>(c.N1, L1.w, ws);
+        if (c.N1 > 0) k_weight_sums<<<256, 256, 0, E.stream>>>(c.N1, L1.d4, ws);
         CF_CHECK(hipGetLastError());
         double h[2];
         CF_CHECK(hipMemcpyAsync(h, ws, sizeof h, hipMemcpyDeviceToHost, E.stream));
@@ -1885,7 +1893,7 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         double* ws = (double*)E.arena.get("bwsums", sizeof(double) * 2 * ncat);
         fill_u64(ws, 2 * (int64_t)ncat);
         for (int k = 0; k < ncat; k++)
-            if (ND[k] > 0) k_weight_sums<<<64, 256, 0, E.stream>>>(ND[k], hl[k].w, ws + 2 * k);
+            if (ND[k] > 0) k_weight_sums<<<64, 256, 0, E.stream>>>(ND[k], hl[k].d4, ws + 2 * k);
         CF_CHECK(hipGetLastError());
         CF_CHECK(hipMemcpyAsync(wsums.data(), ws, sizeof(double) * 2 * ncat, hipMemcpyDeviceToHost, E.stream));
     }
@@ -2089,7 +2097,7 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
     }
     const int64_t nngb_cap = (int64_t)(2 * refine_cap[0] + 1) * (2 * refine_cap[1] + 1) * (2 * refine_cap[2] + 1);
     const int64_t cand_cap = ncap * nngb_cap;
-    if (ncap * kSlabs >= (int64_t)INT32_MAX || cand_cap >= (int64_t)INT32_MAX) {
+    if (ncap >= (int64_t)INT32_MAX || cand_cap >= (int64_t)INT32_MAX) {
         fprintf(stderr, "Error: the graph batch's grid capacity exceeds the engine's 32-bit indexing\n");
         return EXIT_FAILURE;
     }
@@ -2152,24 +2160,23 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
     unsigned short* d_lut = (unsigned short*)G.alloc(sizeof(unsigned short) * lut.size());
     CF_CHECK(hipMemcpy(d_edges, rupp_sqr.data(), sizeof(double) * nbin, hipMemcpyHostToDevice));
     CF_CHECK(hipMemcpy(d_lut, lut.data(), sizeof(unsigned short) * lut.size(), hipMemcpyHostToDevice));
-    const int64_t nb_cap = ncap * kSlabs;
+    const int64_t nb_cap = ncap;
     std::vector<DevLattice> tmpl(ncat);
-    std::vector<int*> bucket(ncat), counts(ncat), fillb(ncat);
+    std::vector<int*> bucket(ncat), rank(ncat), idx(ncat), big(ncat), counts(ncat);
     for (int k = 0; k < ncat; k++) {
         const int64_t n = ND[k];
         DevLattice& L = tmpl[k];
         memset(&L, 0, sizeof L);
-        L.x = (double*)G.alloc(sizeof(double) * (size_t)n);
-        L.y = (double*)G.alloc(sizeof(double) * (size_t)n);
-        L.z = (double*)G.alloc(sizeof(double) * (size_t)n);
-        L.w = need_w ? (double*)G.alloc(sizeof(double) * (size_t)n) : nullptr;
         L.d4 = (double4*)G.alloc(sizeof(double4) * (size_t)(n + kQPad));
         L.q = (uint2*)G.alloc(sizeof(uint2) * (size_t)(n + kQPad));
         L.bstart = (int*)G.alloc(sizeof(int) * (size_t)(nb_cap + 1));
         L.bounds = (double*)G.alloc(sizeof(double) * 6 * (size_t)ncap);
+        L.gbox = (double*)G.alloc(sizeof(double) * 6 * (size_t)(n / kGroup + ncap + 1));
         bucket[k] = (int*)G.alloc(sizeof(int) * (size_t)(n + 1));
+        rank[k] = (int*)G.alloc(sizeof(int) * (size_t)(n + 1));
+        idx[k] = (int*)G.alloc(sizeof(int) * (size_t)(n + 1));
+        big[k] = (int*)G.alloc(sizeof(int) * (size_t)(n / kSmallCell + 1));
         counts[k] = (int*)G.alloc(sizeof(int) * (size_t)(nb_cap + 1));
-        fillb[k] = (int*)G.alloc(sizeof(int) * (size_t)(nb_cap + 1));
     }
     // scheduler buffers (as launch_tuned's)
     const int sched = E.sched_kind;
@@ -2227,32 +2234,38 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         const int64_t n = ND[k];
         const BgCat* ck = G.cats + k;
         fill_i(counts[k], nb_cap + 1, 0);
-        fill_i(fillb[k], nb_cap + 1, 0);
+        fill_i(big[k], 1, 0);
         const unsigned nblk = (unsigned)((n + 255) / 256);
         if (n > 0) {
             if (esize == 4)
                 k_bg_bucket_count<float><<<nblk, 256, 0, st>>>(n, (const float*)X[k], (const float*)Y[k],
-                                                               (const float*)Z[k], ck, bucket[k], counts[k], oob);
+                                                               (const float*)Z[k], ck, bucket[k], rank[k],
+                                                               counts[k], oob);
             else
                 k_bg_bucket_count<double><<<nblk, 256, 0, st>>>(n, (const double*)X[k], (const double*)Y[k],
-                                                                (const double*)Z[k], ck, bucket[k], counts[k], oob);
+                                                                (const double*)Z[k], ck, bucket[k], rank[k],
+                                                                counts[k], oob);
         }
         scan.run(counts[k], tmpl[k].bstart, nb_cap, st);
-        if (n > 0) {
-            if (esize == 4)
-                k_bg_scatter<float><<<nblk, 256, 0, st>>>(n, (const float*)X[k], (const float*)Y[k],
-                                                          (const float*)Z[k], (const float*)(need_w ? W[k] : nullptr),
-                                                          ck, bucket[k], tmpl[k].bstart, fillb[k], tmpl[k].x,
-                                                          tmpl[k].y, tmpl[k].z, tmpl[k].w, tmpl[k].d4, tmpl[k].q);
-            else
-                k_bg_scatter<double><<<nblk, 256, 0, st>>>(n, (const double*)X[k], (const double*)Y[k],
-                                                           (const double*)Z[k],
-                                                           (const double*)(need_w ? W[k] : nullptr), ck, bucket[k],
-                                                           tmpl[k].bstart, fillb[k], tmpl[k].x, tmpl[k].y,
-                                                           tmpl[k].z, tmpl[k].w, tmpl[k].d4, tmpl[k].q);
+        if (n > 0) k_index_scatter<<<nblk, 256, 0, st>>>(n, bucket[k], rank[k], tmpl[k].bstart, idx[k]);
+        const unsigned sb = (unsigned)((ncap + 3) / 4), bb = (unsigned)std::min<int64_t>(n / kSmallCell, 2 * E.ncu);
+        const void* wk = need_w ? W[k] : nullptr;
+        if (esize == 4) {
+            k_bg_build_small<float><<<sb, 256, 0, st>>>((const float*)X[k], (const float*)Y[k], (const float*)Z[k],
+                                                        (const float*)wk, ck, tmpl[k], idx[k], rank[k], big[k]);
+            if (bb > 0)
+                k_bg_build_big<float><<<bb, kBigThreads, 0, st>>>((const float*)X[k], (const float*)Y[k],
+                                                                  (const float*)Z[k], (const float*)wk, ck, tmpl[k],
+                                                                  idx[k], rank[k], big[k]);
+        } else {
+            k_bg_build_small<double><<<sb, 256, 0, st>>>((const double*)X[k], (const double*)Y[k],
+                                                         (const double*)Z[k], (const double*)wk, ck, tmpl[k], idx[k],
+                                                         rank[k], big[k]);
+            if (bb > 0)
+                k_bg_build_big<double><<<bb, kBigThreads, 0, st>>>((const double*)X[k], (const double*)Y[k],
+                                                                   (const double*)Z[k], (const double*)wk, ck,
+                                                                   tmpl[k], idx[k], rank[k], big[k]);
         }
-        k_bg_cell_bounds<<<(unsigned)((ncap + 3) / 4), 256, 0, st>>>(ck, tmpl[k].bstart, tmpl[k].x, tmpl[k].y,
-                                                                      tmpl[k].z, tmpl[k].bounds);
         // neighbour-cell pairs, appended to the list at cp_off[k]
         k_bg_cellpair_flag<<<(unsigned)((cand_cap + 255) / 256), 256, 0, st>>>(ck, cand_cap, tmpl[k].bstart,
                                                                                 tmpl[k].bounds, flags);
@@ -2260,7 +2273,7 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         k_bg_cp_offset<<<1, 64, 0, st>>>(k, pos, cand_cap, G.cp_off, G.pairs_cap, G.fail);
         k_bg_cellpair_emit<<<(unsigned)std::min<int64_t>((cand_cap + 255) / 256, 1024), 256, 0, st>>>(
             ck, cand_cap, tmpl[k].bstart, tmpl[k].bounds, pos, G.cp_off, k, G.pairs_cap, cps, G.tested);
-        if (need_w && n > 0) k_weight_sums<<<64, 256, 0, st>>>(n, tmpl[k].w, G.ws + 2 * k);
+        if (need_w && n > 0) k_weight_sums<<<64, 256, 0, st>>>(n, tmpl[k].d4, G.ws + 2 * k);
     }
     k_oob_flag<<<1, 64, 0, st>>>(oob, G.fail, kBgFailOob);
     // work list as launch_tuned builds it (cost order, heavy cell pairs first

@@ -2,12 +2,14 @@
 //
 // Device pipeline of one countpairs* call:
 //   k_minmax / k_minmax_final     data extent              (reference gridlink_utils.c.src:52-70)
-//   k_bucket_count                cell index + z-slab per particle, bucket histogram
+//   k_bucket_count                cell index per particle, cell histogram
 //                                                          (gridlink_impl.c.src:162-201)
-//   k_scan_*                      exclusive prefix sum of the bucket histogram
-//   k_scatter                     counting-sort scatter into SoA arrays in HBM (FP64 + quantized
-//                                 cell-local positions for the integer pair filter)
-//   k_cell_bounds                 per-cell bounding boxes  (gridlink_impl.c.src:292-316)
+//   k_scan_*                      exclusive prefix sum of the cell histogram
+//   k_index_scatter               particle indices in cell order
+//   k_build_small / _big          per cell: Hilbert order, records in HBM (FP64 + quantized
+//                                 cell-local positions for the integer pair filter), the
+//                                 bounding boxes of the cell (gridlink_impl.c.src:292-316)
+//                                 and of its groups
 //   k_cellpair_flag / _emit       neighbour-cell work list with periodic wraps and
 //                                 min-separation culling   (gridlink_impl.c.src:439-625)
 //   k_pairs_plain                 FP64 pair kernel, one workgroup per cell pair
@@ -103,48 +105,55 @@ __device__ __forceinline__ uint2 quantize_pos(double dx, double dy, double dz, d
     return make_uint2(((unsigned)qx & 0xffffu) | ((unsigned)qy << 16), (unsigned)qz);
 }
 
-// Cell index exactly as the reference computes it (gridlink_impl.c.src:167-178),
-// followed by the z-slab inside the cell.
-__device__ __forceinline__ int cell_and_slab(const GridArgs& g, double X, double Y, double Z, int* cell, int* oob)
+// Cell index exactly as the reference computes it (gridlink_impl.c.src:167-178).
+__device__ __forceinline__ int cell_of(const GridArgs& g, double X, double Y, double Z, int* oob)
 {
     int ix = (int)((X - g.xmin) * g.xinv);
     int iy = (int)((Y - g.ymin) * g.yinv);
-    const double zr = (Z - g.zmin) * g.zinv;
-    int iz = (int)zr;
+    int iz = (int)((Z - g.zmin) * g.zinv);
     if (ix > g.nx - 1) ix--;
     if (iy > g.ny - 1) iy--;
     if (iz > g.nz - 1) iz--;
     *oob = ix < 0 || ix >= g.nx || iy < 0 || iy >= g.ny || iz < 0 || iz >= g.nz;
-    *cell = (ix * g.ny + iy) * g.nz + iz;
-    int s = (int)((zr - (double)iz) * kSlabs);
-    s = s < 0 ? 0 : (s > kSlabs - 1 ? kSlabs - 1 : s);
-    return s;
+    return (ix * g.ny + iy) * g.nz + iz;
 }
 
+// The particle's cell and its rank among the cell's particles (the order of
+// the atomics, so any order), which the index scatter needs no second atomic for.
 template <typename T>
 __device__ __forceinline__ void bucket_count_one(int64_t i, const T* __restrict__ X, const T* __restrict__ Y,
                                                  const T* __restrict__ Z, const GridArgs& g, int* __restrict__ bucket,
-                                                 int* __restrict__ counts, unsigned long long* __restrict__ oob_count)
+                                                 int* __restrict__ rank, int* __restrict__ counts,
+                                                 unsigned long long* __restrict__ oob_count)
 {
-    int c, oob;
-    const int s = cell_and_slab(g, (double)X[i], (double)Y[i], (double)Z[i], &c, &oob);
+    int oob;
+    const int c = cell_of(g, (double)X[i], (double)Y[i], (double)Z[i], &oob);
     if (oob) {
         atomicAdd(oob_count, 1ull);
         bucket[i] = -1;
         return;
     }
-    const int b = c * kSlabs + s;
-    bucket[i] = b;
-    atomicAdd(&counts[b], 1);
+    bucket[i] = c;
+    rank[i] = atomicAdd(&counts[c], 1);
 }
 
 template <typename T>
 __global__ void k_bucket_count(int64_t n, const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-                               GridArgs g, int* __restrict__ bucket, int* __restrict__ counts,
-                               unsigned long long* __restrict__ oob_count)
+                               GridArgs g, int* __restrict__ bucket, int* __restrict__ rank,
+                               int* __restrict__ counts, unsigned long long* __restrict__ oob_count)
 {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) bucket_count_one(i, X, Y, Z, g, bucket, counts, oob_count);
+    if (i < n) bucket_count_one(i, X, Y, Z, g, bucket, rank, counts, oob_count);
+}
+
+// Particle indices in cell order.
+__global__ void k_index_scatter(int64_t n, const int* __restrict__ bucket, const int* __restrict__ rank,
+                                const int* __restrict__ bstart, int* __restrict__ idx)
+{
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int b = bucket[i];
+    if (b >= 0) idx[bstart[b] + rank[i]] = (int)i;  // b < 0: outside the grid, reported by the host
 }
 
 // Exclusive scan over int32 counts, three phases, 1024 items per block.
@@ -197,59 +206,127 @@ __global__ void k_scan_add(int64_t n, int* __restrict__ out, const int* __restri
         if (base + k < n) out[base + k] += add;
 }
 
-template <typename T>
-__device__ __forceinline__ void scatter_one(int64_t i, const T* __restrict__ X, const T* __restrict__ Y,
-                                            const T* __restrict__ Z, const T* __restrict__ W, const GridArgs& g,
-                                            const int* __restrict__ bucket, const int* __restrict__ bstart,
-                                            int* __restrict__ fill, double* __restrict__ x, double* __restrict__ y,
-                                            double* __restrict__ z, double* __restrict__ w, double4* __restrict__ d4,
-                                            uint2* __restrict__ q)
+// Position of (x, y, z), b bits each, on the 3-D Hilbert curve (J. Skilling,
+// "Programming the Hilbert curve", 2004: inverse undo of the excess work, then
+// Gray encoding).
+__device__ __forceinline__ unsigned hilbert3(unsigned x, unsigned y, unsigned z, int b)
 {
-    const int b = bucket[i];
-    if (b < 0) return;  // outside the grid: counted by k_bucket_count, reported by the host
-    const int pos = bstart[b] + atomicAdd(&fill[b], 1);
-    const double xv = (double)X[i], yv = (double)Y[i], zv = (double)Z[i];
-    x[pos] = xv;
-    y[pos] = yv;
-    z[pos] = zv;
-    const double wv = W ? (double)W[i] : 0.0;
-    if (W) w[pos] = wv;
-    d4[pos] = make_double4(xv, yv, zv, wv);
-    const int c = b / kSlabs;
-    const int iz = c % g.nz, ixy = c / g.nz, iy = ixy % g.ny, ix = ixy / g.ny;
-    const double ox = g.xmin + ix * g.xbs, oy = g.ymin + iy * g.ybs, oz = g.zmin + iz * g.zbs;
-    q[pos] = quantize_pos(xv - ox, yv - oy, zv - oz, g.qinv);
-}
-
-template <typename T>
-__global__ void k_scatter(int64_t n, const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-                          const T* __restrict__ W, GridArgs g, const int* __restrict__ bucket,
-                          const int* __restrict__ bstart, int* __restrict__ fill,
-                          double* __restrict__ x, double* __restrict__ y, double* __restrict__ z,
-                          double* __restrict__ w, double4* __restrict__ d4, uint2* __restrict__ q)
-{
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) scatter_one(i, X, Y, Z, W, g, bucket, bstart, fill, x, y, z, w, d4, q);
-}
-
-// Per-cell bounding boxes, one wave per cell (lanes stride over the cell's
-// particles, then a shuffle reduction; min/max are exact, so the order of the
-// reduction does not matter). Empty cells get (+DBL_MAX, -DBL_MAX).
-__device__ __forceinline__ void cell_bounds_one(int64_t c, const int* __restrict__ bstart,
-                                                const double* __restrict__ x, const double* __restrict__ y,
-                                                const double* __restrict__ z, double* __restrict__ bounds)
-{
-    const int lane = threadIdx.x & 63;
-    double b[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
-    const int e = bstart[(c + 1) * kSlabs];
-    for (int k = bstart[c * kSlabs] + lane; k < e; k += 64) {
-        b[0] = x[k] < b[0] ? x[k] : b[0];
-        b[1] = x[k] > b[1] ? x[k] : b[1];
-        b[2] = y[k] < b[2] ? y[k] : b[2];
-        b[3] = y[k] > b[3] ? y[k] : b[3];
-        b[4] = z[k] < b[4] ? z[k] : b[4];
-        b[5] = z[k] > b[5] ? z[k] : b[5];
+    unsigned v[3] = {x, y, z};
+    for (int k = b - 1; k > 0; k--) {
+        const unsigned q = 1u << k, m = q - 1u;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const unsigned t = (v[0] ^ v[d]) & m;
+            const bool up = (v[d] & q) != 0;
+            v[0] ^= up ? m : t;
+            if (d > 0) v[d] ^= up ? 0u : t;
+        }
     }
+    v[1] ^= v[0];
+    v[2] ^= v[1];
+    unsigned t = 0;
+    for (int k = b - 1; k > 0; k--)
+        if (v[2] & (1u << k)) t ^= (1u << k) - 1u;
+    unsigned h = 0;
+    for (int k = b - 1; k >= 0; k--)
+        h = (h << 3) | ((((v[0] ^ t) >> k) & 1u) << 2) | ((((v[1] ^ t) >> k) & 1u) << 1) | (((v[2] ^ t) >> k) & 1u);
+    return h;
+}
+
+// Cells up to kSmallCell particles are sorted by one wave each, larger ones by
+// a workgroup of kBigThreads.
+constexpr int kSmallCell = 512;
+constexpr int kSmallBins = 512;
+constexpr int kBigBins = 4096;
+constexpr int kBigThreads = 1024;
+constexpr int kMaxSegments = 8;
+
+template <int NT>
+__device__ __forceinline__ void build_sync()
+{
+    __threadfence_block();
+    if (NT == 64)
+        __builtin_amdgcn_wave_barrier();
+    else
+        __syncthreads();
+}
+
+// Orders the particles of cell c along a Hilbert curve through the cell (a
+// counting sort over up to MAXBINS sub-cells in LDS, `hist`), so that runs of
+// consecutive particles are compact, and writes their FP64 records, quantized
+// cell-local positions, the cell's bounding box and the bounding boxes of its
+// groups of kGroup. A cell longer in z than in x and y is cut into cubic
+// segments along z, one curve each. Two gathers of the particles' coordinates
+// (key, placement) instead of one pass that keeps them in registers: the
+// second hits L2, and any cell size takes the same code. The whole of NT
+// threads (`tid` in it) works on one cell; `red` holds 6 NT / 64 doubles (NT > 64).
+template <typename T, int NT, int MAXBINS>
+__device__ __forceinline__ void build_cell(int64_t c, int tid, const T* __restrict__ X, const T* __restrict__ Y,
+                                           const T* __restrict__ Z, const T* __restrict__ W, const GridArgs& g,
+                                           const int* __restrict__ bstart, const int* __restrict__ idx,
+                                           int* __restrict__ keys, double4* d4, uint2* __restrict__ q,
+                                           double* __restrict__ bounds, double* __restrict__ gbox, int* hist,
+                                           double* red)
+{
+    const int s = bstart[c], n = bstart[c + 1] - s;
+    const int lane = tid & 63;
+    double b[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
+    const int ic = (int)c, iz = ic % g.nz, ixy = ic / g.nz, iy = ixy % g.ny, ix = ixy / g.ny;
+    const double ox = g.xmin + ix * g.xbs, oy = g.ymin + iy * g.ybs, oz = g.zmin + iz * g.zbs;
+    if (n > 0) {
+        const double side = fmax(g.xbs, g.ybs);
+        int nseg = side > 0 ? (int)fmin((double)kMaxSegments, g.zbs / side + 0.5) : 1;
+        nseg = nseg < 1 ? 1 : nseg;
+        int nb = 0;
+        while (nb < 5 && (nseg << (3 * (nb + 1))) <= min(MAXBINS, 2 * n)) nb++;
+        const int bins = nseg << (3 * nb), top = (1 << nb) - 1;
+        const double scale = (double)(1 << nb);
+        for (int k = tid; k < bins; k += NT) hist[k] = 0;
+        build_sync<NT>();
+        for (int k = tid; k < n; k += NT) {
+            const int i = idx[s + k];
+            const double xv = (double)X[i], yv = (double)Y[i], zv = (double)Z[i];
+            b[0] = xv < b[0] ? xv : b[0];
+            b[1] = xv > b[1] ? xv : b[1];
+            b[2] = yv < b[2] ? yv : b[2];
+            b[3] = yv > b[3] ? yv : b[3];
+            b[4] = zv < b[4] ? zv : b[4];
+            b[5] = zv > b[5] ? zv : b[5];
+            const int hx = (int)fmin(fmax((xv - ox) * g.xinv * scale, 0.0), (double)top);
+            const int hy = (int)fmin(fmax((yv - oy) * g.yinv * scale, 0.0), (double)top);
+            const int zt = (nseg << nb) - 1;
+            const int hz = (int)fmin(fmax((zv - oz) * g.zinv * scale * nseg, 0.0), (double)zt);
+            const int key = ((hz >> nb) << (3 * nb)) + (int)hilbert3(hx, hy, hz & top, nb);
+            keys[s + k] = key;
+            atomicAdd(&hist[key], 1);
+        }
+        build_sync<NT>();
+        // exclusive scan of the bins by the first wave
+        if (tid < 64) {
+            int carry = 0;
+            for (int k0 = 0; k0 < bins; k0 += 64) {
+                const int k = k0 + lane;
+                const int v = k < bins ? hist[k] : 0;
+                int incl = v;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int t = __shfl_up(incl, o, 64);
+                    if (lane >= o) incl += t;
+                }
+                if (k < bins) hist[k] = carry + incl - v;
+                carry += __shfl(incl, 63, 64);
+            }
+        }
+        build_sync<NT>();
+        for (int k = tid; k < n; k += NT) {
+            const int i = idx[s + k];
+            const double xv = (double)X[i], yv = (double)Y[i], zv = (double)Z[i];
+            const int pos = s + atomicAdd(&hist[keys[s + k]], 1);
+            d4[pos] = make_double4(xv, yv, zv, W ? (double)W[i] : 0.0);
+            q[pos] = quantize_pos(xv - ox, yv - oy, zv - oz, g.qinv);
+        }
+    }
+    // cell bounds (min / max are exact, so the order of the reduction does not
+    // matter); empty cells get (+DBL_MAX, -DBL_MAX)
     for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
         for (int d = 0; d < 6; d += 2) {
@@ -258,23 +335,101 @@ __device__ __forceinline__ void cell_bounds_one(int64_t c, const int* __restrict
             b[d + 1] = hi > b[d + 1] ? hi : b[d + 1];
         }
     }
-    if (lane == 0)
+    if (NT > 64) {
+        if (lane == 0)
+            for (int d = 0; d < 6; d++) red[(tid >> 6) * 6 + d] = b[d];
+        __syncthreads();
+        if (tid < 6) {
+            double v = red[tid];
+            for (int w = 1; w < NT / 64; w++) {
+                const double t = red[w * 6 + tid];
+                v = (tid & 1) ? (t > v ? t : v) : (t < v ? t : v);
+            }
+            bounds[c * 6 + tid] = v;
+        }
+    } else if (lane == 0) {
         for (int d = 0; d < 6; d++) bounds[c * 6 + d] = b[d];
+    }
+    // group boxes, kGroup lanes per group, from the records just written
+    build_sync<NT>();
+    const int64_t g0 = group_index(s, c);
+    for (int gk = tid / kGroup; gk * kGroup < n; gk += NT / kGroup) {
+        const int k = gk * kGroup + (tid & (kGroup - 1));
+        double e[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
+        if (k < n) {
+            const double4 r = d4[s + k];
+            // a NaN coordinate leaves the empty range (it is in no pair)
+            e[0] = fmin(e[0], r.x); e[1] = fmax(e[1], r.x);
+            e[2] = fmin(e[2], r.y); e[3] = fmax(e[3], r.y);
+            e[4] = fmin(e[4], r.z); e[5] = fmax(e[5], r.z);
+        }
+        for (int o = kGroup / 2; o > 0; o >>= 1) {
+#pragma unroll
+            for (int d = 0; d < 6; d += 2) {
+                e[d] = fmin(e[d], __shfl_xor(e[d], o, 64));
+                e[d + 1] = fmax(e[d + 1], __shfl_xor(e[d + 1], o, 64));
+            }
+        }
+        const int d = tid & (kGroup - 1);
+        const double v = d == 0 ? e[0] : d == 1 ? e[1] : d == 2 ? e[2] : d == 3 ? e[3] : d == 4 ? e[4] : e[5];
+        if (d < 6) gbox[(g0 + gk) * 6 + d] = v;
+    }
 }
 
-__global__ void k_cell_bounds(int64_t ncells, const int* __restrict__ bstart, const double* __restrict__ x,
-                              const double* __restrict__ y, const double* __restrict__ z, double* __restrict__ bounds)
+// One wave per cell; cells above kSmallCell particles are left to
+// k_build_big, listed at big[1 ...] with their number at big[0].
+template <typename T>
+__device__ __forceinline__ void build_small(int64_t ncells, const T* X, const T* Y, const T* Z, const T* W,
+                                            const GridArgs& g, const int* bstart, const int* idx, int* keys,
+                                            double4* d4, uint2* q, double* bounds, double* gbox, int* big)
 {
-    const int64_t c = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-    if (c < ncells) cell_bounds_one(c, bstart, x, y, z, bounds);  // uniform per wave
+    __shared__ int hist[4][kSmallBins];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t c = blockIdx.x * (int64_t)(blockDim.x >> 6) + wave;
+    if (c >= ncells) return;  // uniform per wave
+    if (bstart[c + 1] - bstart[c] > kSmallCell) {
+        if (lane == 0) big[1 + atomicAdd(big, 1)] = (int)c;
+        return;
+    }
+    build_cell<T, 64, kSmallBins>(c, lane, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, hist[wave], nullptr);
+}
+template <typename T>
+__device__ __forceinline__ void build_big(const T* X, const T* Y, const T* Z, const T* W, const GridArgs& g,
+                                          const int* bstart, const int* idx, int* keys, double4* d4, uint2* q,
+                                          double* bounds, double* gbox, const int* big)
+{
+    __shared__ int hist[kBigBins];
+    __shared__ double red[6 * kBigThreads / 64];
+    const int nbig = big[0];
+    for (int t = blockIdx.x; t < nbig; t += gridDim.x) {
+        build_cell<T, kBigThreads, kBigBins>(big[1 + t], threadIdx.x, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds,
+                                             gbox, hist, red);
+        __syncthreads();
+    }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void k_build_small(int64_t ncells, const T* X, const T* Y, const T* Z, const T* W,
+                                                     GridArgs g, const int* bstart, const int* idx, int* keys,
+                                                     double4* d4, uint2* q, double* bounds, double* gbox, int* big)
+{
+    build_small(ncells, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, big);
+}
+template <typename T>
+__global__ __launch_bounds__(kBigThreads) void k_build_big(const T* X, const T* Y, const T* Z, const T* W, GridArgs g,
+                                                           const int* bstart, const int* idx, int* keys, double4* d4,
+                                                           uint2* q, double* bounds, double* gbox, const int* big)
+{
+    build_big(X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, big);
 }
 
-__global__ void k_weight_sums(int64_t n, const double* __restrict__ w, double* __restrict__ out)
+// Sums of the weights and of their squares over the grid-ordered records.
+__global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double* __restrict__ out)
 {
     double s = 0, s2 = 0;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        s += w[i];
-        s2 += w[i] * w[i];
+        const double w = d4[i].w;
+        s += w;
+        s2 += w * w;
     }
     for (int o = 32; o > 0; o >>= 1) {
         s += __shfl_xor(s, o, 64);
@@ -309,7 +464,7 @@ struct NgbArgs {
 
 __device__ __forceinline__ int64_t cell_count(const int* bstart, int64_t c)
 {
-    return (int64_t)bstart[(c + 1) * kSlabs] - bstart[c * kSlabs];
+    return (int64_t)bstart[c + 1] - bstart[c];
 }
 
 // Evaluates neighbour k of primary cell icell in the reference's loop order
@@ -670,18 +825,19 @@ __global__ __launch_bounds__(128) void k_pairs_plain(PairParams P, DevLattice L1
     }
     const CellPairRec cp = cps[blockIdx.x];
     const int mode = P.mode;
-    const int i0 = L1.bstart[(int64_t)cp.c1 * kSlabs], i1 = L1.bstart[(int64_t)(cp.c1 + 1) * kSlabs];
-    const int j0 = L2.bstart[(int64_t)cp.c2 * kSlabs], j1 = L2.bstart[(int64_t)(cp.c2 + 1) * kSlabs];
+    const int i0 = L1.bstart[cp.c1], i1 = L1.bstart[cp.c1 + 1];
+    const int j0 = L2.bstart[cp.c2], j1 = L2.bstart[cp.c2 + 1];
     for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
         ITerms t = {};
-        i_terms(P, mode, cp, L1.x[i], L1.y[i], L1.z[i], &t);
+        const double4 pi = L1.d4[i];
+        i_terms(P, mode, cp, pi.x, pi.y, pi.z, &t);
         if (t.skip) continue;
-        const double wi = P.need_w ? L1.w[i] : 0.0;
         const int jstart = cp.same ? i + 1 : j0;
         for (int j = jstart; j < j1; j++) {
             double sep = 0;
-            const int slot = replay_pair(P, mode, t, cp.same, 1, L2.x[j], L2.y[j], L2.z[j], e, &sep);
-            if (slot >= 0) hist_add(P, h, slot, sep, P.need_w ? wi * L2.w[j] : 0.0);
+            const double4 pj = L2.d4[j];
+            const int slot = replay_pair(P, mode, t, cp.same, 1, pj.x, pj.y, pj.z, e, &sep);
+            if (slot >= 0) hist_add(P, h, slot, sep, P.need_w ? pi.w * pj.w : 0.0);
         }
     }
     if (GH) return;
@@ -696,13 +852,14 @@ template __global__ void k_pairs_plain<true>(PairParams, DevLattice, DevLattice,
 // ------------------------------------------------- tuned pair kernel
 // Work item: (cell pair, chunk of <= 64 consecutive primary particles).
 // Each wave pulls work items from a device counter until the list is exhausted.
-// Lane l holds primary particle i0+l. The secondary particles of the cell pair,
-// restricted to the z-slabs the chunk can reach, are read with scalar loads: the
-// index is wave-uniform, so a secondary lands in scalar registers that every
-// lane's vector instructions read directly (no per-lane load, no broadcast
-// instruction). Two paths per work item:
-//  * dense (every pair of the cell pair is inside the separation range): each
-//    (i, j) is decided in FP64 in lockstep from a 32-byte (x, y, z, w) record;
+// Lane l holds primary particle i0+l. The secondary particles of the cell pair
+// come in groups of kGroup with a bounding box each; the lanes test 64 groups at
+// a time against the chunk's box, and runs of groups within reach are read with
+// scalar loads: the index is wave-uniform, so a secondary lands in scalar
+// registers that every lane's vector instructions read directly (no per-lane
+// load, no broadcast instruction). Two paths per group:
+//  * dense (enough of its pairs are in range): each (i, j) is decided in FP64 in
+//    lockstep from a 32-byte (x, y, z, w) record;
 //  * sparse: an integer test on quantized cell-local positions (packed 16-bit
 //    differences, one dot-product instruction per pair), with thresholds that
 //    provably pass every pair the FP64 test can accept, rejects the pairs that
@@ -711,6 +868,7 @@ template __global__ void k_pairs_plain<true>(PairParams, DevLattice, DevLattice,
 // Either way every counted pair is decided by the reference's FP64 arithmetic.
 constexpr int kQueues = 8;          // work sub-queues (one counter each)
 constexpr int kCounterStride = 32;  // ints between sub-queue counters (128 B)
+constexpr int kFewGroups = 2;       // secondary windows up to this many groups are not box-tested
 constexpr int kBlockJ = 4;          // secondaries per scalar load of the sparse path
 // Survivor buffer per wave: entries (j << 6) | lane at [head, tail). Drains take
 // 64 * DP entries from the head (DP survivors per lane: 1, or 2 with both pairs'
@@ -723,11 +881,8 @@ constexpr int kBlockJ = 4;          // secondaries per scalar load of the sparse
 // furthest write is 127 + 64 (kBlockJ - 1) + 127 < kQueueAlloc.
 constexpr int kCompactAt = 128;
 constexpr int kQueueAlloc = kCompactAt + 64 + 64 * (kBlockJ - 1) + 127;
-// Queue entries hold secondary indices relative to the start of the window
-// being scanned, ((j - jbase) << 6) | lane in 32 bits: a secondary window longer
-// than P.max_window (2^25 by default, a multiple of kBlockJ) is scanned in
-// consecutive sub-windows of that length, with the queue drained at the end of
-// each.
+// Queue entries hold secondary indices relative to the first one of the 64
+// groups being scanned, ((j - jbase) << 6) | lane.
 
 // Read-only particle data seen through the constant address space: loads with a
 // wave-uniform index become scalar loads.
@@ -888,7 +1043,8 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
             const CellPairRec* c = fresh(cpp);
             const DevLattice* l1 = fresh(l1p);
             ITerms t = {};
-            i_terms(P, MODE, *c, l1->x[i], l1->y[i], l1->z[i], &t);
+            const double4 p = l1->d4[i];
+            i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
             if (t.skip || zj <= t.target || dz >= t.max_dz) return;
         }
         const int k = lut_kbin<FL>(P, S, key);
@@ -912,7 +1068,8 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
         const CellPairRec* c = fresh(cpp);
         const DevLattice* l1 = fresh(l1p);
         ITerms t = {};
-        i_terms(P, MODE, *c, l1->x[i], l1->y[i], l1->z[i], &t);
+        const double4 p = l1->d4[i];
+        i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
         if (is2d) {
             if (!c->same && (t.skip || zj <= t.target)) return;
         } else {
@@ -1163,7 +1320,6 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
     const int lane = lane_id();
     const int i0 = __builtin_amdgcn_readfirstlane(it.i0), i1 = __builtin_amdgcn_readfirstlane(it.i1);
     const int flags = __builtin_amdgcn_readfirstlane(it.flags);
-    const int dense = Pi.dense_mode == 1 ? 1 : (Pi.dense_mode == 2 ? 0 : (flags & kItemDense));
     // with P.dense_stride, dense cross-cell items take strided primaries (a
     // whole-cell sample per wave, spreading the lanes' pairs over more
     // histogram slots); else 64 consecutive ones
@@ -1185,57 +1341,26 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
         zpos = pi.z + wrap.z;
         wi = pi.w;
     }
-    // secondary z-slabs this chunk can reach
-    const int iz2 = c2 % L2.nz;
-    const double zlo = wave_min_d(ivalid ? zpos : DBL_MAX) - Pi.zreach - Pi.slab_margin;
-    const double zhi = wave_max_d(ivalid ? zpos : -DBL_MAX) + Pi.zreach + Pi.slab_margin;
-    int jlo, jhi;
-    {
-        const int64_t cb = (int64_t)c2 * kSlabs;
-        double flo = floor(((zlo - L2.zmin) * L2.zinv - (double)iz2) * kSlabs);
-        double fhi = floor(((zhi - L2.zmin) * L2.zinv - (double)iz2) * kSlabs);
-        if (L2.zinv == 0.0) { flo = 0.0; fhi = kSlabs - 1; }
-        if (fhi < 0.0 || flo > (double)(kSlabs - 1)) {
-            jlo = jhi = 0;
-        } else {
-            const int slo = flo < 0.0 ? 0 : (int)flo;
-            const int shi = fhi > (double)(kSlabs - 1) ? kSlabs - 1 : (int)fhi;
-            jlo = L2.bstart[cb + slo];
-            jhi = L2.bstart[cb + shi + 1];
-        }
-    }
-    if (same && jlo < i0 + 1) jlo = i0 + 1;
-    jlo = __builtin_amdgcn_readfirstlane(jlo);
-    jhi = __builtin_amdgcn_readfirstlane(jhi);
+    // groups of kGroup secondaries of the cell; same cell: from the chunk's own on
+    const int s2 = __builtin_amdgcn_readfirstlane(L2.bstart[c2]), e2 = __builtin_amdgcn_readfirstlane(L2.bstart[c2 + 1]);
+    int glo = same ? (i0 - s2) / kGroup : 0, ghi = (e2 - s2 + kGroup - 1) / kGroup;
     {
         const int nparts = __builtin_amdgcn_readfirstlane(it.nparts);
-        if (nparts > 1 && jhi > jlo) {
+        if (nparts > 1) {
             const int part = __builtin_amdgcn_readfirstlane(it.part);
-            const int64_t len = jhi - jlo;
-            const int a = jlo + (int)(len * part / nparts), b = jlo + (int)(len * (part + 1) / nparts);
-            jlo = a;
-            jhi = b;
+            const int64_t len = ghi - glo;
+            const int a = glo + (int)(len * part / nparts), b = glo + (int)(len * (part + 1) / nparts);
+            glo = a;
+            ghi = b;
         }
     }
-
-    if (jhi <= jlo) return;
-
-    if (dense) {
-        // FP64 lockstep; the secondary record is a scalar load (d4 is padded, so
-        // the look-ahead load of j + 1 stays inside the array)
-        KDouble* ds = (KDouble*)(const void*)d4_2;
-        double4 cur = kload_d4(ds, jlo);
-        for (int j = jlo; j < jhi; j++) {
-            const double4 nxt = kload_d4(ds, j + 1);
-            exact_pair<MODE, R2F, GH, FL>(P, cpp, l1p, i, j > ilim, xpos, ypos, zpos, wi, cur.x, cur.y, cur.z,
-                                          fl_w<FL>(P) ? cur.w : 0.0, S);
-            cur = nxt;
-        }
-        return;
-    }
-
-    // sparse: quantize the wave's primaries relative to the secondary cell
-    const int ixy2 = c2 / L2.nz, iy2 = ixy2 % L2.ny, ix2 = ixy2 / L2.ny;
+    if (ghi <= glo) return;
+    // with at most kFewGroups groups the cell pair's own dense estimate decides
+    // (the cell pair list has culled by the cells' boxes)
+    const bool few = ghi - glo <= kFewGroups;
+    const double* gb2 = L2.gbox + group_index(s2, c2) * 6;
+    // sparse path: quantize the wave's primaries relative to the secondary cell
+    const int iz2 = c2 % L2.nz, ixy2 = c2 / L2.nz, iy2 = ixy2 % L2.ny, ix2 = ixy2 / L2.ny;
     const double ox = L2.xmin + ix2 * L2.xbs, oy = L2.ymin + iy2 * L2.ybs, oz = L2.zmin + iz2 * L2.zbs;
     // a lane without a primary gets (qx, qy) = (-32768, -32768): every difference
     // to a secondary (0 <= q <= kQMax) wraps to |dq| >= 32768 - kQMax per axis, so
@@ -1258,37 +1383,132 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
         prim[lane] = make_double4(xpos, ypos, zpos, wi);
         __builtin_amdgcn_wave_barrier();
     }
+    KDouble* ds = (KDouble*)(const void*)d4_2;
     KUint* qs = (KUint*)(const void*)L2.q;
-    const int max_window = Pi.max_window;
     constexpr int kDrain = 64 * DP;
-    for (int wlo = jlo; wlo < jhi; wlo += max_window) {
-        const int whi = jhi - wlo > max_window ? wlo + max_window : jhi;
-        QBlock a = qload(qs, wlo);
-        int jb = wlo;
-        while (jb < whi) {
-            if (same)
-                jb = qscan<MODE, true, kDrain>(f, qs, jb, whi, a, qe, head, tail, wlo);
-            else
-                jb = qscan<MODE, false, kDrain>(f, qs, jb, whi, a, qe, head, tail, wlo);
-            if (jb < whi && jb + kBlockJ > whi && tail - head < kDrain) {
-                // the last, partial block
-                if (same)
-                    qblock<MODE, true, true>(f, a, jb, whi - jb, qe, tail, wlo);
-                else
-                    qblock<MODE, false, true>(f, a, jb, whi - jb, qe, tail, wlo);
-                jb = whi;
+    for (int g0 = glo; g0 < ghi; g0 += 64) {
+        // lane l tests group g0 + l against the chunk's box: out of reach,
+        // dense (enough of its pairs in range), or sparse
+        unsigned long long mdense, msparse;
+        if (few) {
+            const unsigned long long ml = ~0ull >> (64 - (ghi - glo));
+            const bool dns = Pi.dense_mode == 0 ? (flags & kItemDense) != 0 : Pi.dense_mode == 1;
+            mdense = dns ? ml : 0ull;
+            msparse = dns ? 0ull : ml;
+        } else {
+            // the chunk's bounding box (wrapped): the union of its groups' boxes, or
+            // the cell's for strided primaries (recomputed per 64 groups: kept
+            // across the scans it costs 12 registers there)
+            double A[6];
+            {
+                const int c1 = cp.c1;
+                const int s1 = __builtin_amdgcn_readfirstlane(L1.bstart[c1]);
+                KDouble* ub = (KDouble*)(const void*)(stride > 0 ? L1.bounds + (int64_t)c1 * 6
+                                                                 : L1.gbox + (group_index(s1, c1) + (i0 - s1) / kGroup) * 6);
+                const int ng = stride > 0 ? 1 : (i1 - i0 + kGroup - 1) / kGroup;
+#pragma unroll
+                for (int d = 0; d < 6; d++) A[d] = ub[d];
+                for (int k = 1; k < ng; k++)
+#pragma unroll
+                    for (int d = 0; d < 6; d += 2) {
+                        A[d] = fmin(A[d], ub[6 * k + d]);
+                        A[d + 1] = fmax(A[d + 1], ub[6 * k + d + 1]);
+                    }
+                A[0] += wrap.x; A[1] += wrap.x;
+                A[2] += wrap.y; A[3] += wrap.y;
+                A[4] += wrap.z; A[5] += wrap.z;
             }
-            while (tail - head >= kDrain) {
+            const bool have = g0 + lane < ghi;
+            const double* bx = gb2 + (int64_t)(have ? g0 + lane : glo) * 6;
+            const double x0 = bx[0], x1 = bx[1], y0 = bx[2], y1 = bx[3], z0 = bx[4], z1 = bx[5];
+            const double nx = fmax(fmax(x0 - A[1], A[0] - x1), 0.0), ny = fmax(fmax(y0 - A[3], A[2] - y1), 0.0),
+                         nz = fmax(fmax(z0 - A[5], A[4] - z1), 0.0);
+            const double fx = fmax(x1 - A[0], A[1] - x0), fy = fmax(y1 - A[2], A[3] - y0),
+                         fz = fmax(z1 - A[4], A[5] - z0);
+            constexpr bool is2d = MODE == MODE_RPPI || MODE == MODE_WP;
+            const double near2 = is2d ? nx * nx + ny * ny : nx * nx + ny * ny + nz * nz;
+            const double far2 = is2d ? fx * fx + fy * fy : fx * fx + fy * fy + fz * fz;
+            // the margins cover the rounding of the pairs' own separations
+            const bool live = have && near2 <= P.sqr_rmax * (1.0 + 1e-9) && nz <= P.zreach * (1.0 + 1e-9) + P.box_margin;
+            double num = P.sqr_rmax - near2, den = far2 - near2;
+            bool dns = num >= (double)P.dense_frac * den;
+            if (is2d) {
+                // times the share of |dz| below pimax
+                const double zn = fmax(P.pimax - nz, 0.0), zd = fz - nz;
+                dns = fmin(num, den) * fmin(zn, zd) >= (double)P.dense_frac * (den * zd);
+            }
+            if (Pi.dense_mode != 0) dns = Pi.dense_mode == 1;
+            if (stride > 0) dns = true;
+            const unsigned long long ml = __builtin_amdgcn_ballot_w64(live);
+            mdense = ml & __builtin_amdgcn_ballot_w64(dns);
+            msparse = ml & ~mdense;
+        }
+        while (mdense) {
+            // a run of consecutive dense groups: FP64 lockstep; the secondary
+            // record is a scalar load (d4 is padded, so the look-ahead load of
+            // j + 1 stays inside the array)
+            const int g = __builtin_ctzll(mdense);
+            const unsigned long long rest = ~(mdense >> g);
+            const int run = rest ? __builtin_ctzll(rest) : 64;
+            mdense = g + run < 64 ? mdense & (~0ull << (g + run)) : 0ull;
+            int j = s2 + (g0 + g) * kGroup;
+            const int je = min(j + run * kGroup, e2);
+            double4 cur = kload_d4(ds, j);
+            for (; j < je; j++) {
+                const double4 nxt = kload_d4(ds, j + 1);
+                exact_pair<MODE, R2F, GH, FL>(P, cpp, l1p, i, j > ilim, xpos, ypos, zpos, wi, cur.x, cur.y, cur.z,
+                                              fl_w<FL>(P) ? cur.w : 0.0, S);
+                cur = nxt;
+            }
+        }
+        // sparse runs: filter into the queue and drain full rounds; what is left
+        // is drained after the batch's last run, so that queue entries can hold
+        // j relative to the batch's first secondary
+        const int jbase = s2 + g0 * kGroup;
+        int jb = 0, jhi = 0;  // the run being scanned
+        QBlock a = {};        // its block at jb
+        bool last = msparse == 0;
+        while (!last) {
+            if (jb >= jhi) {
+                if (msparse) {
+                    const int g = __builtin_ctzll(msparse);
+                    const unsigned long long rest = ~(msparse >> g);
+                    const int run = rest ? __builtin_ctzll(rest) : 64;
+                    msparse = g + run < 64 ? msparse & (~0ull << (g + run)) : 0ull;
+                    jb = s2 + (g0 + g) * kGroup;
+                    jhi = min(jb + run * kGroup, e2);
+                    a = qload(qs, jb);
+                } else {
+                    last = true;
+                }
+            }
+            if (!last) {
+                if (same)
+                    jb = qscan<MODE, true, kDrain>(f, qs, jb, jhi, a, qe, head, tail, jbase);
+                else
+                    jb = qscan<MODE, false, kDrain>(f, qs, jb, jhi, a, qe, head, tail, jbase);
+                if (jb < jhi && jb + kBlockJ > jhi && tail - head < kDrain) {
+                    // the last, partial block
+                    if (same)
+                        qblock<MODE, true, true>(f, a, jb, jhi - jb, qe, tail, jbase);
+                    else
+                        qblock<MODE, false, true>(f, a, jb, jhi - jb, qe, tail, jbase);
+                    jb = jhi;
+                }
+            }
+            while (tail - head >= (last ? 1u : (unsigned)kDrain)) {
+                const unsigned nd = min(tail - head, (unsigned)kDrain);
                 __builtin_amdgcn_wave_barrier();
                 if (DP == 2)
                     drain_queue2<MODE, R2F, GH, FL>(P, cp, cpp, l1p, d4_1, d4_2, wrap, i0, istride, qe, prim, head,
-                                                kDrain, wlo, S);
+                                                    (int)nd, jbase, S);
                 else
                     drain_queue<MODE, R2F, GH, FL>(P, cp, cpp, l1p, d4_1, d4_2, wrap, i0, istride, qe, prim, head,
-                                               kDrain, wlo, S);
+                                                   (int)nd, jbase, S);
                 __builtin_amdgcn_wave_barrier();
-                head += kDrain;
+                head += nd;
             }
+            if (last) head = tail = 0;
             if (head >= kCompactAt) {
                 // move the < kDrain waiting entries to the front
                 const unsigned n = tail - head;
@@ -1307,17 +1527,6 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
                 tail = n;
             }
         }
-        if (tail != head) {
-            __builtin_amdgcn_wave_barrier();
-            if (DP == 2)
-                drain_queue2<MODE, R2F, GH, FL>(P, cp, cpp, l1p, d4_1, d4_2, wrap, i0, istride, qe, prim, head,
-                                            (int)(tail - head), wlo, S);
-            else
-                drain_queue<MODE, R2F, GH, FL>(P, cp, cpp, l1p, d4_1, d4_2, wrap, i0, istride, qe, prim, head,
-                                           (int)(tail - head), wlo, S);
-            __builtin_amdgcn_wave_barrier();
-        }
-        head = tail = 0;
     }
 }
 
@@ -1608,7 +1817,7 @@ __global__ void k_emit_chunks(int ncp, const int* __restrict__ order, const Cell
     const double* bd2 = lats[batch ? cp.pad : 1].bounds;
     double maxsep2;
     const int dense = cp_dense(P, cp, bd1 + (int64_t)cp.c1 * 6, bd2 + (int64_t)cp.c2 * 6, &maxsep2);
-    const int s = bs1[(int64_t)cp.c1 * kSlabs], e = bs1[(int64_t)(cp.c1 + 1) * kSlabs];
+    const int s = bs1[cp.c1], e = bs1[cp.c1 + 1];
     const int parts = nparts ? nparts[t] : 1;
     int o = off[t];
     const int nch = (e - s + 63) / 64;
