@@ -85,7 +85,7 @@ struct PairParams {
     double inv_d2, sqr_mu_max;
     double max_all_dz_same;  // same-cell z window (DD/xi/s_mu)
     double xwrap, ywrap, zwrap;
-    double near_r2, near_dz; // edge windows below which pruning replay is skipped
+    double near_lo2, near_lodz; // squared separation and |dz| below which pruning replay is skipped
     double zreach;           // largest |dz| of a counted pair
     double box_margin;       // slack of the group boxes' z test
     // bin lookup: slot count of edges below the 1/16-octave bucket of (float)r^2
@@ -116,10 +116,11 @@ constexpr int kMaxParts = 32;
 // Per-cell-pair features of the cost model (computed on the device).
 constexpr int kNumFeatures = 10;
 // f0 log2(1+N1)       f1 log2(1+N2)        f2 log2(chunks of 64 primaries)
-// f3 same cell        f4 dense (bounding boxes entirely in range)
+// f3 same cell        f4 estimated share of the pairs in range
 // f5 min separation^2 / rmax^2              f6 max separation^2 / rmax^2 (<= 8)
-// f7 fraction of the secondary cell's z extent within z reach of the primaries
+// f7 share of the (primary, secondary) group pairs within reach
 // f8 projected (rp, pi) mode                f9 log2(1 + N2 * f7)
+// (f4, f7: from a sample of the groups' bounding boxes)
 
 // Cost-ordered work lists: heavy cell pairs are bucketed by log2 cost, descending.
 constexpr float kCostTop = 48.0f;        // log2 cost mapped to bucket 0

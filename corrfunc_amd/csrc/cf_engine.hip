@@ -774,8 +774,8 @@ static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, con
     P.zwrap = wrap[2];
     // Edge windows: the reference's pruning tests can only reject pairs whose
     // separation lies within a few ulps of the coordinate scale below rmax / pimax.
-    P.near_r2 = 1e-9 * P.sqr_rmax + 1e-9 * rmax * coord_scale;
-    P.near_dz = 1e-9 * pimax + 1e-9 * coord_scale;
+    P.near_lo2 = P.sqr_rmax - (1e-9 * P.sqr_rmax + 1e-9 * rmax * coord_scale);
+    P.near_lodz = P.pimax - (1e-9 * pimax + 1e-9 * coord_scale);
     P.zreach = (is2d || mode == MODE_SMU) ? pimax : sqrt(P.sqr_rmax);
     P.box_margin = 1e-7 * (coord_scale + cs);
 
@@ -1569,7 +1569,7 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
             P.sqr_rmax = mode == MODE_RPPI_MOCKS ? rmax * rmax + pimax * pimax : rupp_sqr[nbin - 1];
             P.max_all_dz_same = sqrt(P.sqr_rmax - 0.0 - 0.0);
             P.zreach = sqrt(P.sqr_rmax);
-            P.near_r2 = 1e-9 * P.sqr_rmax + 1e-9 * max_sep * coord_scale;
+            P.near_lo2 = P.sqr_rmax - (1e-9 * P.sqr_rmax + 1e-9 * max_sep * coord_scale);
         }
         set_quant_filter(L1, P);
         set_quant_filter(L2, P);

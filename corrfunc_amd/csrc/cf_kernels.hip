@@ -898,17 +898,23 @@ __device__ __forceinline__ uint2 kload_u2(KUint* p, int j)
 }
 typedef short short2v __attribute__((ext_vector_type(2)));
 
-// sqrt(r2) to ~1e-14 relative: the hardware FP32 square root (about 1 ulp)
-// refined by one Newton step in FP64.
-__device__ __forceinline__ double fast_sqrt(double r2)
+// sqrt(r2) to ~1e-14 relative from y = the hardware FP32 reciprocal square root
+// of f = (float)r2: s = f y, one FP32 Newton step (to about half an ulp of FP32),
+// one in FP64. One transcendental (a quarter of the FMA rate), shared with the mu
+// bin, instead of a square root and a reciprocal. Lanes below 1e-30 take sqrt; the
+// test is one branch of the whole wave.
+__device__ __forceinline__ double fast_sqrt(double r2, float f, float y)
 {
-    const float f = (float)r2;
-    if (!(f > 1e-30f)) return sqrt(r2);
-    const float s = __builtin_amdgcn_sqrtf(f);
+    const float h = 0.5f * y, s0 = f * y;
+    const float s = fmaf(fmaf(-s0, s0, f), h, s0);
     const double sd = (double)s;
-    const double res = fma(-sd, sd, r2);
-    const double half_inv = 0.5 * (double)__builtin_amdgcn_rcpf(s);
-    return fma(res, half_inv, sd);
+    double r = fma(fma(-sd, sd, r2), (double)h, sd);
+    if (__builtin_amdgcn_ballot_w64(!(f > 1e-30f))) {
+        double q = sqrt(r2);
+        asm volatile("" : "+v"(q));  // keeps the branch: the compiler would compute q always and select
+        r = f > 1e-30f ? r : q;
+    }
+    return r;
 }
 
 // Histogram of one workgroup of the tuned kernel, replicated R ways with layout
@@ -921,7 +927,7 @@ struct KernelLds {
     unsigned long long* np;
     double* avg;
     double* w;
-    int rmask;                 // R - 1
+    int rshift;                // log2 R
     int lane_copy;             // lane & (R - 1)
     const double* e;           // rupp_sqr[0..nbin-1]
     const unsigned short* lut; // bin lookup
@@ -962,35 +968,65 @@ __device__ __forceinline__ constexpr bool float_index_of()
     return (MODE == MODE_RPPI && R2F == RP_FMA) || (MODE == MODE_SMU && R2F == R2_FMA_DX_DY_DZ);
 }
 
-// Adds a counted pair (slot, squared separation r2, weight product) to the histogram.
+// Adds a counted pair (slot, squared separation r2, weight product) to the
+// histogram; f = (float)r2, y its reciprocal square root.
 template <bool GH, int FL>
-__device__ __forceinline__ void hist_pair(const PairParams& P, KernelLds& S, int slot, double r2, double wprod)
+__device__ __forceinline__ void hist_pair(const PairParams& P, KernelLds& S, int slot, double r2, float f, float y,
+                                          double wprod)
 {
     if (GH) {
         atomicAdd(&S.gnp[slot], 1ull);
-        if (fl_avg<FL>(P)) atomicAdd(&S.gavg[slot], fast_sqrt(r2));
+        if (fl_avg<FL>(P)) atomicAdd(&S.gavg[slot], fast_sqrt(r2, f, y));
         if (fl_w<FL>(P)) atomicAdd(&S.gw[slot], wprod);
         return;
     }
-    const int a = slot * (S.rmask + 1) + S.lane_copy;
+    const int a = (slot << S.rshift) + S.lane_copy;
     atomicAdd(&S.np[a], 1ull);
-    if (fl_avg<FL>(P)) atomicAdd(&S.avg[a], fast_sqrt(r2));
+    if (fl_avg<FL>(P)) atomicAdd(&S.avg[a], fast_sqrt(r2, f, y));
     if (fl_w<FL>(P)) atomicAdd(&S.w[a], wprod);
 }
 
 // Number of edges e[0..nbin-2] <= r2 (the reference's top-down bin search,
-// countpairs_kernels.c.src:982-993, for non-decreasing edges): start from the
-// lookup table's lower bound for the 1/16-octave bucket of (float)r2 and step up.
+// countpairs_kernels.c.src:982-993, for non-decreasing edges), for e[0] <= r2 <
+// e[nbin-1]: start from the lookup table's lower bound for the 1/16-octave bucket
+// of f = (float)r2 and step up. (The table ends above the bucket of e[nbin-1], so
+// only its start needs a clamp: e[0] may be 0.) 0 only for unsorted edges.
 template <int FL>
-__device__ __forceinline__ int lut_kbin(const PairParams& P, const KernelLds& S, double r2)
+__device__ __forceinline__ int lut_kbin(const PairParams& P, const KernelLds& S, double r2, float f)
 {
     if (!fl_lut1<FL>(P) && !P.sorted_edges) return find_kbin(S.e, P.nbin, 0, r2);
-    int idx = (int)(__float_as_uint((float)r2) >> 19) - P.lut_base;
-    idx = idx < 0 ? 0 : (idx >= P.lut_n ? P.lut_n - 1 : idx);
+    const unsigned idx = __builtin_elementwise_sub_sat(__float_as_uint(f) >> 19, (unsigned)P.lut_base);
     int k = S.lut[idx];
     if (fl_lut1<FL>(P)) return k + (S.e[k] <= r2 ? 1 : 0);  // e[nbin-1] = rmax^2 > r2
     while (k < P.nbin - 1 && S.e[k] <= r2) k++;
     return k;
+}
+
+// slot of bin k, column m (24-bit multiply: an LDS histogram has fewer slots).
+template <bool GH>
+__device__ __forceinline__ int slot_of(const PairParams& P, int k, int m)
+{
+    return GH ? k * (P.n2 + 1) + m : (int)__umul24((unsigned)k, (unsigned)(P.n2 + 1)) + m;
+}
+
+// Whether the integer part of an FP32 estimate t with error below 1e-6 (t + 1) is
+// certain (false for NaN and infinities).
+__device__ __forceinline__ bool column_sure(float t)
+{
+    return fabsf(__builtin_amdgcn_fractf(t) - 0.5f) <= fmaf(-1e-6f, t, 0.499999f);
+}
+
+// a / b, correctly rounded for operands whose quotient and reciprocal are normal
+// (Markstein: two Newton steps on the hardware reciprocal, then one on the
+// quotient with its exact remainder); the general division also scales and fixes
+// up the ranges that squared comoving distances do not reach.
+__device__ __forceinline__ double quotient(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
 }
 
 // FP64 separation in the rounding order R2F of the reference kernel being replayed.
@@ -1035,11 +1071,40 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
     constexpr bool onsky = MODE == MODE_RPPI_MOCKS || MODE == MODE_SMU_MOCKS;
     const double dx = xj - xpos, dy = yj - ypos, dz = zj - zpos;
     if (onsky) {
+        // as los_split, with the pi / mu column from an FP32 estimate: each factor
+        // rounded once and the hardware roots (1 ulp) put t within 7e-7 of its value,
+        // so its integer part is the reference's unless t is within 1e-6 (t + 1) of an
+        // integer; only those pairs take the FP64 root (and, for mu, the quotient)
+        const double parx = xpos + xj, pary = ypos + yj, parz = zpos + zj;
+        const double sqr_s = dx * dx + dy * dy + dz * dz;
+        const double s_dot_l = parx * dx + pary * dy + parz * dz;
+        const double sqr_l = parx * parx + pary * pary + parz * parz;
+        const double sqr_s_dot_l = s_dot_l * s_dot_l;
+        const double sqr_lim = P.sqr_mu_max;
+        bool in = ok && sqr_s < P.sqr_rmax;
         double key;
         int j2;
-        if (!ok || !los_split(P, MODE, xpos, ypos, zpos, xj, yj, zj, &key, &j2)) return;
+        if (MODE == MODE_RPPI_MOCKS) {
+            if (!(in && sqr_s_dot_l < sqr_l * sqr_lim)) return;
+            const double sqr_par = quotient(sqr_s_dot_l, sqr_l);
+            key = sqr_s - sqr_par;
+            if (!(key < P.sqr_rpmax && key >= P.sqr_rmin)) return;
+            const float t = __builtin_amdgcn_sqrtf((float)sqr_par) * (float)P.inv_d2;
+            j2 = (int)t;
+            if (!column_sure(t)) j2 = sqr_par >= sqr_lim ? P.n2 : (int)(sqrt(sqr_par) * P.inv_d2);
+        } else {
+            if (!(in && sqr_s >= P.sqr_rmin)) return;
+            key = sqr_s;
+            const float t = fabsf((float)s_dot_l) * __builtin_amdgcn_rsqf((float)sqr_l) *
+                            __builtin_amdgcn_rsqf((float)sqr_s) * (float)P.inv_d2;
+            j2 = (int)fminf(t, (float)P.n2);
+            if (!column_sure(t)) {
+                const double sqr_mu = sqr_s_dot_l / (sqr_l * sqr_s);
+                j2 = sqr_mu >= sqr_lim ? P.n2 : (int)(sqrt(sqr_mu) * P.inv_d2);
+            }
+        }
         // pruning replay for pairs near the 3-D limit (the 3-D kernels' rules)
-        if (sep2<R2F>(dx, dy, dz) >= P.sqr_rmax - P.near_r2) {
+        if (sep2<R2F>(dx, dy, dz) >= P.near_lo2) {
             const CellPairRec* c = fresh(cpp);
             const DevLattice* l1 = fresh(l1p);
             ITerms t = {};
@@ -1047,22 +1112,23 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
             i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
             if (t.skip || zj <= t.target || dz >= t.max_dz) return;
         }
-        const int k = lut_kbin<FL>(P, S, key);
-        if (k == 0) return;
-        hist_pair<GH, FL>(P, S, k * (P.n2 + 1) + j2, key, wi * wj);
+        const float f = (float)key;
+        const int k = lut_kbin<FL>(P, S, key, f);
+        if (!fl_lut1<FL>(P) && k == 0) return;
+        hist_pair<GH, FL>(P, S, slot_of<GH>(P, k, j2), key, f, __builtin_amdgcn_rsqf(f), wi * wj);
         return;
     }
     const double sqr_dz = dz * dz;
     const double r2 = sep2<R2F>(dx, dy, dz);
     const double adz = fabs(dz);
     bool in = ok && r2 < P.sqr_rmax && r2 >= P.sqr_rmin;
-    if (is2d) in = in && dz > -P.pimax && dz < P.pimax;
+    if (is2d) in = in && adz < P.pimax;
     if (MODE == MODE_SMU) in = in && sqr_dz < r2 * P.sqr_mu_max;
     if (!in) return;
     // The reference's pruning tests (per-particle minimum separation, z window)
     // can only reject pairs within a few ulps of the coordinate scale of rmax or
     // pimax; only such pairs replay them.
-    const bool near = r2 >= P.sqr_rmax - P.near_r2 || (MODE != MODE_DD && MODE != MODE_XI && adz >= P.pimax - P.near_dz);
+    const bool near = r2 >= P.near_lo2 || (MODE != MODE_DD && MODE != MODE_XI && adz >= P.near_lodz);
     if (near) {
         // the cell pair record and the primary set, loaded here
         const CellPairRec* c = fresh(cpp);
@@ -1077,30 +1143,17 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
         }
     }
     const bool findex = FL < 0 ? P.float_index != 0 : float_index_of<MODE, R2F>();
-    int k;
-    if (fl_lut1<FL>(P) || P.sorted_edges) {
-        int idx = (int)(__float_as_uint((float)r2) >> 19) - P.lut_base;
-        idx = idx < 0 ? 0 : (idx >= P.lut_n ? P.lut_n - 1 : idx);
-        k = S.lut[idx];
-        if (fl_lut1<FL>(P)) {
-            // at most one edge above lut[idx] can lie below r2 (e[nbin-1] = rmax^2 > r2)
-            k += S.e[k] <= r2 ? 1 : 0;
-        } else if (k < P.nbin - 1 && S.e[k] <= r2) {
-            k++;
-            while (k < P.nbin - 1 && S.e[k] <= r2) k++;
-        }
-    } else {
-        k = find_kbin(S.e, P.nbin, 0, r2);
-    }
-    if (k == 0) return;
+    const float f = (float)r2;
+    const int k = lut_kbin<FL>(P, S, r2, f);
+    if (!fl_lut1<FL>(P) && k == 0) return;
+    const float y = MODE == MODE_SMU || fl_avg<FL>(P) ? __builtin_amdgcn_rsqf(f) : 0.0f;
     int slot = k;
     if (MODE == MODE_RPPI) {
         if (findex) {
             slot = (int)((double)k * (double)(P.n2 + 1) + adz * P.inv_d2);
         } else {
             int pb = (int)(adz * P.inv_d2);
-            pb = pb > P.n2 ? P.n2 : pb;
-            slot = k * (P.n2 + 1) + pb;
+            slot = slot_of<GH>(P, k, pb > P.n2 ? P.n2 : pb);
         }
     } else if (MODE == MODE_SMU) {
         // mu bin from an FP32 estimate t ~ mu * inv_dmu: |dz|, s^2 and inv_dmu
@@ -1108,26 +1161,22 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
         // ulp) and two products put t within 4e-7 * t of the reference's FP64
         // value, so its integer part is the reference's unless t lies within
         // 1e-6 * (t + 1) of an integer; only those pairs (and non-finite
-        // estimates, clamped to 1e9) compute mu = sqrt(dz^2 / s^2) in FP64 as the
-        // reference does (countpairs_s_mu_kernels.c.src:1154-1171).
-        const float t = fminf((float)adz * __builtin_amdgcn_rsqf((float)r2) * (float)P.inv_d2, 1e9f);
-        const int mbf = (int)t;
-        const float fr = t - (float)mbf;
-        const float tol = 1e-6f * (t + 1.0f);
-        if (fr >= tol && fr <= 1.0f - tol) {
-            slot = k * (P.n2 + 1) + (mbf > P.n2 ? P.n2 : mbf);
+        // estimates) compute mu = sqrt(dz^2 / s^2) in FP64 as the reference does
+        // (countpairs_s_mu_kernels.c.src:1154-1171).
+        const float t = (float)adz * y * (float)P.inv_d2;
+        if (column_sure(t)) {
+            slot = slot_of<GH>(P, k, min((int)t, P.n2));
         } else {
             const double mu = sqrt(sqr_dz / r2);
             if (findex) {
                 slot = (int)((double)k * (double)(P.n2 + 1) + mu * P.inv_d2);
             } else {
-                int mb = (int)(mu * P.inv_d2);
-                mb = mb > P.n2 ? P.n2 : mb;
-                slot = k * (P.n2 + 1) + mb;
+                const int mb = (int)(mu * P.inv_d2);
+                slot = slot_of<GH>(P, k, mb > P.n2 ? P.n2 : mb);
             }
         }
     }
-    hist_pair<GH, FL>(P, S, slot, r2, wi * wj);
+    hist_pair<GH, FL>(P, S, slot, r2, f, y, wi * wj);
 }
 
 // Decides up to 64 queued survivors (entries ((j - jbase) << 6) | lane) in FP64.
@@ -1588,7 +1637,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(DP == 2 ? 
     S.np = np0 + roff;
     S.avg = avg0 + roff;
     S.w = w0 + roff;
-    S.rmask = R - 1;
+    S.rshift = __builtin_ctz(R);
     S.lane_copy = lane & (R - 1);
     S.gnp = g_np;
     S.gavg = g_avg;

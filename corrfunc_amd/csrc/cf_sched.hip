@@ -34,29 +34,51 @@ __global__ void k_cp_features(int ncp, const CellPairRec* __restrict__ cps, cons
     const double* b1 = A.bounds + (int64_t)cp.c1 * 6;
     const double* b2 = B.bounds + (int64_t)cp.c2 * 6;
     double maxsep2;
-    const int dense = cp_dense(P, cp, b1, b2, &maxsep2);
+    cp_dense(P, cp, b1, b2, &maxsep2);
     const int is2d = P.mode == MODE_RPPI || P.mode == MODE_WP;
     const double minsep2 = cp.mdx * cp.mdx + cp.mdy * cp.mdy + (is2d ? 0.0 : cp.mdz * cp.mdz);
-    const double oz = cp.wz * P.zwrap;
-    const double zlo = b1[4] + oz - P.zreach, zhi = b1[5] + oz + P.zreach;
-    const double ext2 = b2[5] - b2[4];
-    double zfrac = 1.0;
-    if (ext2 > 0) {
-        const double ov = fmin(zhi, b2[5]) - fmax(zlo, b2[4]);
-        zfrac = fmin(1.0, fmax(0.0, ov / ext2));
-    }
+    // what the pair kernel's group tests will find, on up to 16 x 16 evenly spaced
+    // (group of primaries, group of secondaries) pairs: the share within reach and
+    // the estimated share of pairs in range
+    const int g1 = ((int)n1 + kGroup - 1) / kGroup, g2 = ((int)n2 + kGroup - 1) / kGroup;
+    const int d1 = (g1 + 15) / 16, d2 = (g2 + 15) / 16;
+    const double* x1 = A.gbox + group_index(A.bstart[cp.c1], cp.c1) * 6;
+    const double* x2 = B.gbox + group_index(B.bstart[cp.c2], cp.c2) * 6;
+    const double off[3] = {cp.wx * P.xwrap, cp.wy * P.ywrap, cp.wz * P.zwrap};
+    int ntest = 0;
+    double reach = 0.0, range = 0.0;
+    for (int a = 0; a < g1; a += d1)
+        for (int b = 0; b < g2; b += d2) {
+            double near[3], far[3];
+            for (int d = 0; d < 3; d++) {
+                const double lo1 = x1[6 * (int64_t)a + 2 * d] + off[d], hi1 = x1[6 * (int64_t)a + 2 * d + 1] + off[d];
+                const double lo2 = x2[6 * (int64_t)b + 2 * d], hi2 = x2[6 * (int64_t)b + 2 * d + 1];
+                near[d] = fmax(fmax(lo2 - hi1, lo1 - hi2), 0.0);
+                far[d] = fmax(hi2 - lo1, hi1 - lo2);
+            }
+            const double lo = near[0] * near[0] + near[1] * near[1] + (is2d ? 0.0 : near[2] * near[2]);
+            const double hi = far[0] * far[0] + far[1] * far[1] + (is2d ? 0.0 : far[2] * far[2]);
+            ntest++;
+            if (lo < P.sqr_rmax && near[2] <= P.zreach) {
+                reach += 1.0;
+                double f = hi > P.sqr_rmax ? (P.sqr_rmax - lo) / (hi - lo) : 1.0;
+                if (far[2] > P.zreach) f *= (P.zreach - near[2]) / (far[2] - near[2]);
+                range += f;
+            }
+        }
+    const double nt = (double)(ntest > 0 ? ntest : 1);
     const double inv = P.sqr_rmax > 0 ? 1.0 / P.sqr_rmax : 0.0;
     float* f = feats + (int64_t)t * kNumFeatures;
     f[0] = (float)log2(1.0 + n1);
     f[1] = (float)log2(1.0 + n2);
     f[2] = (float)log2(fmax(1.0, ceil(n1 / 64.0)));
     f[3] = (float)cp.same;
-    f[4] = (float)dense;
+    f[4] = (float)(range / nt);
     f[5] = (float)fmin(8.0, minsep2 * inv);
     f[6] = (float)fmin(8.0, maxsep2 * inv);
-    f[7] = (float)zfrac;
+    f[7] = (float)(reach / nt);
     f[8] = (float)is2d;
-    f[9] = (float)log2(1.0 + n2 * zfrac);
+    f[9] = (float)log2(1.0 + n2 * reach / nt);
 }
 
 // The plain heuristic: log2 of the number of pairs tested, N1*N2 (N1(N1-1)/2

@@ -37,8 +37,8 @@ _KINDS = {"none": NONE, "heuristic": HEURISTIC, "learned": LEARNED}
 FEATURES = _lib.MODEL_FEATURES
 NPARAM = _lib.MODEL_PARAMS
 NNORM = _lib.MODEL_NORM
-FEATURE_NAMES = ("log2(1+N1)", "log2(1+N2)", "log2(chunks)", "same_cell", "dense", "min_sep2/rmax2",
-                 "max_sep2/rmax2", "z_overlap", "projected", "log2(1+N2*z_overlap)")
+FEATURE_NAMES = ("log2(1+N1)", "log2(1+N2)", "log2(chunks)", "same_cell", "in_range", "min_sep2/rmax2",
+                 "max_sep2/rmax2", "in_reach", "projected", "log2(1+N2*in_reach)")
 
 
 def _fp(a):
