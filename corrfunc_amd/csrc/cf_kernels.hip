@@ -358,10 +358,12 @@ __device__ __forceinline__ void build_cell(int64_t c, int tid, const T* __restri
         double e[6] = {DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX, DBL_MAX, -DBL_MAX};
         if (k < n) {
             const double4 r = d4[s + k];
-            // a NaN coordinate leaves the empty range (it is in no pair)
-            e[0] = fmin(e[0], r.x); e[1] = fmax(e[1], r.x);
-            e[2] = fmin(e[2], r.y); e[3] = fmax(e[3], r.y);
-            e[4] = fmin(e[4], r.z); e[5] = fmax(e[5], r.z);
+            // a particle with a NaN coordinate is in no pair; the unbounded box keeps
+            // its group off the paths that rely on finite separations
+            const bool nan = r.x != r.x || r.y != r.y || r.z != r.z;
+            e[0] = nan ? -DBL_MAX : r.x; e[1] = nan ? DBL_MAX : r.x;
+            e[2] = nan ? -DBL_MAX : r.y; e[3] = nan ? DBL_MAX : r.y;
+            e[4] = nan ? -DBL_MAX : r.z; e[5] = nan ? DBL_MAX : r.z;
         }
         for (int o = kGroup / 2; o > 0; o >>= 1) {
 #pragma unroll
@@ -1355,6 +1357,105 @@ __device__ __forceinline__ int qscan(const QFilter& f, KUint* qs, int jb, int jh
     }
 }
 
+// Next run of consecutive groups of the mask m (nonzero; cleared from it): the
+// secondaries [j, je) of a cell whose group 0 of the mask starts at jbase.
+__device__ __forceinline__ void next_run(unsigned long long& m, int jbase, int jend, int& j, int& je)
+{
+    const int g = __builtin_ctzll(m);
+    const unsigned long long rest = ~(m >> g);
+    const int run = rest ? __builtin_ctzll(rest) : 64;
+    m = g + run < 64 ? m & (~0ull << (g + run)) : 0ull;
+    j = jbase + g * kGroup;
+    je = min(j + run * kGroup, jend);
+}
+
+// The path of 1-D counts (no sums) for groups whose separations from the chunk
+// fall into at most kMaxRegBins bins: bins k0 .. k0 + NB - 1, the last without an
+// upper edge unless `touch`, which says that its upper edge is rmax. Every (i, j)
+// is decided in FP64 in lockstep as on the dense path, but the bin comes from NB
+// compares that count in registers until the groups of this bin range are done: no
+// lookup (two dependent LDS reads) and no LDS atomic per pair. (With sums it loses:
+// the accumulators spill the rest of the kernel's registers, and a root, a masked
+// add per bin and sum cost what the lookup and the atomics do.)
+constexpr int kMaxRegBins = 4;
+template <int MODE, int R2F, int NB>
+__device__ __forceinline__ void reg_groups(const PairParams& P, const CellPairRec* cpp, const DevLattice* l1p, int i,
+                                           bool ivalid, double xpos, double ypos, double zpos, KDouble* ds,
+                                           unsigned long long m, int jbase, int jend, int k0, bool touch,
+                                           KernelLds& S)
+{
+    double e[NB];
+    unsigned cnt[NB];  // cumulative: pairs below e[b]
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        e[b] = b < NB - 1 || touch ? S.e[min(k0 + b, P.nbin - 1)] : DBL_MAX;
+        if (!ivalid) e[b] = -1.0;  // no pair of a lane without a primary
+        cnt[b] = 0;
+    }
+    auto decide = [&](double xj, double yj, double zj) {
+        const double dx = xj - xpos, dy = yj - ypos, dz = zj - zpos;
+        double r2 = sep2<R2F>(dx, dy, dz);
+        if (touch) {
+            const bool near = r2 >= P.near_lo2 && r2 < P.sqr_rmax;
+            if (__builtin_amdgcn_ballot_w64(near)) {
+                if (near) {
+                    // the reference's pruning tests (see exact_pair)
+                    const CellPairRec* c = fresh(cpp);
+                    const DevLattice* l1 = fresh(l1p);
+                    ITerms t = {};
+                    const double4 p = l1->d4[i];
+                    i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
+                    const bool out = MODE == MODE_WP ? !c->same && (t.skip || zj <= t.target)
+                                                     : t.skip || zj <= t.target || dz >= t.max_dz;
+                    if (out) r2 = P.sqr_rmax;  // in no bin
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; b++) cnt[b] += r2 < e[b] ? 1u : 0u;
+    };
+    // two records per step, loaded one step ahead (the next run's first two after
+    // a run's last), at 32-bit offsets from the batch's first record: the scalar
+    // unit, which issues the loads and the loop, would bound a simpler loop
+    // (2M points, counts, 14 % per launch; d4 is padded)
+    typedef const __attribute__((address_space(4))) char KChar;
+    KChar* base = (KChar*)(ds + 4 * (int64_t)jbase);
+    auto rec = [&](unsigned o) { return kload_d4((KDouble*)(base + o), 0); };
+    int j, je;
+    next_run(m, 0, jend - jbase, j, je);
+    unsigned o = (unsigned)j * 32u;
+    double4 a0 = rec(o), a1 = rec(o + 32u);
+    for (;;) {
+        const unsigned oe = (unsigned)je * 32u;
+        const bool more = m != 0;
+        unsigned no = o;
+        if (more) {
+            next_run(m, 0, jend - jbase, j, je);
+            no = (unsigned)j * 32u;
+        }
+        for (;;) {
+            const unsigned on = o + 64u < oe ? o + 64u : no;
+            const double4 b0 = rec(on), b1 = rec(on + 32u);
+            decide(a0.x, a0.y, a0.z);
+            o += 32u;
+            if (o < oe) {
+                decide(a1.x, a1.y, a1.z);
+                o += 32u;
+            }
+            a0 = b0;
+            a1 = b1;
+            if (o >= oe) break;
+        }
+        if (!more) break;
+        o = no;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const unsigned n = cnt[b] - (b > 0 ? cnt[b > 0 ? b - 1 : 0] : 0u);
+        if (k0 + b > 0 && n) atomicAdd(&S.np[((k0 + b) << S.rshift) + S.lane_copy], (unsigned long long)n);
+    }
+}
+
 // One work item of the tuned kernel (see the comment above kQueues).
 template <int MODE, int R2F, bool GH, int DP, int FL>
 __device__ __forceinline__ void process_item(const PairParams& P, const DevLattice* l1p, const DevLattice* l2p,
@@ -1382,9 +1483,10 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
     const double3 wrap = make_double3(cp.wx * Pi.xwrap, cp.wy * Pi.ywrap, cp.wz * Pi.zwrap);
     const double4* d4_1 = L1.d4;
     const double4* d4_2 = L2.d4;
-    double xpos = 0, ypos = 0, zpos = 0, wi = 0;
-    if (ivalid) {
-        const double4 pi = d4_1[i];
+    double xpos, ypos, zpos, wi;
+    {
+        // (a lane without a primary holds the chunk's last one)
+        const double4 pi = d4_1[ivalid ? i : i1 - 1];
         xpos = pi.x + wrap.x;
         ypos = pi.y + wrap.y;
         zpos = pi.z + wrap.z;
@@ -1438,7 +1540,9 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
     for (int g0 = glo; g0 < ghi; g0 += 64) {
         // lane l tests group g0 + l against the chunk's box: out of reach,
         // dense (enough of its pairs in range), or sparse
-        unsigned long long mdense, msparse;
+        unsigned long long mdense, msparse, mreg = 0;
+        int keyv = 0;  // bin range of the lane's group: k0 | NB << 16 | touch << 20
+        constexpr bool regs = (MODE == MODE_DD || MODE == MODE_XI || MODE == MODE_WP) && !GH && FL == kFlLut1;
         if (few) {
             const unsigned long long ml = ~0ull >> (64 - (ghi - glo));
             const bool dns = Pi.dense_mode == 0 ? (flags & kItemDense) != 0 : Pi.dense_mode == 1;
@@ -1488,20 +1592,53 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
             }
             if (Pi.dense_mode != 0) dns = Pi.dense_mode == 1;
             if (stride > 0) dns = true;
-            const unsigned long long ml = __builtin_amdgcn_ballot_w64(live);
+            unsigned long long ml = __builtin_amdgcn_ballot_w64(live);
+            if constexpr (regs) {
+                // the group's bin range, from its nearest and farthest separation with
+                // the same margins; not for separations FP32 cannot hold (nor NaN)
+                const double lo = near2 * (1.0 - 1e-9), hi = far2 * (1.0 + 1e-9);
+                const bool touch = !(hi < P.near_lo2);
+                bool ok = live && dns && lo < P.sqr_rmax && far2 < 1e30;
+                if (MODE == MODE_WP) ok = ok && fz * (1.0 + 1e-9) < P.near_lodz;
+                if (same) ok = ok && s2 + (g0 + lane) * kGroup >= i1;  // every j > every i
+                ok = ok && stride == 0 && Pi.dense_mode == 0;
+                if (ok) {
+                    const int k0 = lo < P.sqr_rmin ? 0 : lut_kbin<FL>(P, S, lo, (float)lo);
+                    const int k1 = touch ? P.nbin : (hi < P.sqr_rmin ? 0 : lut_kbin<FL>(P, S, hi, (float)hi));
+                    const int nb = k1 - k0 + (touch ? 0 : 1);
+                    ok = nb <= kMaxRegBins;
+                    keyv = k0 | nb << 16 | (touch ? 1 << 20 : 0);
+                }
+                mreg = __builtin_amdgcn_ballot_w64(ok);
+                ml &= ~mreg;
+            }
             mdense = ml & __builtin_amdgcn_ballot_w64(dns);
             msparse = ml & ~mdense;
+        }
+        if constexpr (regs) {
+            while (mreg) {
+                const int key = __builtin_amdgcn_readlane(keyv, __builtin_ctzll(mreg));
+                const unsigned long long m = mreg & __builtin_amdgcn_ballot_w64(keyv == key);
+                mreg &= ~m;
+                const int k0 = key & 0xffff, nb = (key >> 16) & 15;
+                const bool touch = key >> 20;
+                const int jb0 = s2 + g0 * kGroup;
+                if (nb == 1)
+                    reg_groups<MODE, R2F, 1>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
+                else if (nb == 2)
+                    reg_groups<MODE, R2F, 2>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
+                else if (nb == 3)
+                    reg_groups<MODE, R2F, 3>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
+                else if (nb == 4)
+                    reg_groups<MODE, R2F, 4>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
+            }
         }
         while (mdense) {
             // a run of consecutive dense groups: FP64 lockstep; the secondary
             // record is a scalar load (d4 is padded, so the look-ahead load of
             // j + 1 stays inside the array)
-            const int g = __builtin_ctzll(mdense);
-            const unsigned long long rest = ~(mdense >> g);
-            const int run = rest ? __builtin_ctzll(rest) : 64;
-            mdense = g + run < 64 ? mdense & (~0ull << (g + run)) : 0ull;
-            int j = s2 + (g0 + g) * kGroup;
-            const int je = min(j + run * kGroup, e2);
+            int j, je;
+            next_run(mdense, s2 + g0 * kGroup, e2, j, je);
             double4 cur = kload_d4(ds, j);
             for (; j < je; j++) {
                 const double4 nxt = kload_d4(ds, j + 1);
@@ -1520,12 +1657,7 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
         while (!last) {
             if (jb >= jhi) {
                 if (msparse) {
-                    const int g = __builtin_ctzll(msparse);
-                    const unsigned long long rest = ~(msparse >> g);
-                    const int run = rest ? __builtin_ctzll(rest) : 64;
-                    msparse = g + run < 64 ? msparse & (~0ull << (g + run)) : 0ull;
-                    jb = s2 + (g0 + g) * kGroup;
-                    jhi = min(jb + run * kGroup, e2);
+                    next_run(msparse, jbase, e2, jb, jhi);
                     a = qload(qs, jb);
                 } else {
                     last = true;
