@@ -387,10 +387,6 @@ static void device_scan(const int* in, int* out, int64_t n, const std::string& t
         device_scan(bsum, boff, nblocks, tag, depth + 1);
         k_scan_add<<<(unsigned)nblocks, kScanBlock, 0, E.stream>>>(n, out, boff);
         CF_CHECK(hipGetLastError());
-        // total = boff[nblocks]
-        CF_CHECK(hipMemcpyAsync(out + n, boff + nblocks, sizeof(int), hipMemcpyDeviceToDevice, E.stream));
-    } else {
-        CF_CHECK(hipMemcpyAsync(out + n, bsum, sizeof(int), hipMemcpyDeviceToDevice, E.stream));
     }
 }
 
@@ -531,6 +527,9 @@ static int gridlink_device(const std::string& tag, const GridSpec& g, int64_t n,
     return check_oob(h_oob);
 }
 
+// Workgroups of k_weight_sums: 8 records a thread, at most 512 (two atomics each).
+static unsigned weight_blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(512, n / 2048)); }
+
 // Device work list of neighbour-cell pairs (gridlink_impl.c.src:439-625), in
 // two steps: cellpairs_flag marks the kept (cell, neighbour) candidates and
 // scans them (the count lands at plan.pos[plan.total] on the device);
@@ -583,7 +582,7 @@ static void cellpairs_emit(const CpPlan& cp, CellPairRec* out, double* dtested, 
     Engine& E = eng();
     const unsigned blocks = (unsigned)std::min<int64_t>((cp.total + 255) / 256, 1024);
     k_cellpair_emit<<<blocks, 256, 0, E.stream>>>(cp.a, cp.L1.ncells, cp.nngb, cp.L1.bstart, cp.L2.bstart,
-                                                  cp.L1.bounds, cp.L2.bounds, cp.pos, out, dtested, cat);
+                                                  cp.L1.bounds, cp.L2.bounds, cp.flags, cp.pos, out, dtested, cat);
     CF_CHECK(hipGetLastError());
 }
 
@@ -954,6 +953,58 @@ static const void* tuned_kernel(bool gh, int dp, int fl)
     return nullptr;
 }
 
+// Cell pairs of at most kLightPairs tests go to k_pairs_light when the cell pairs
+// have at most kLightMean tests on average.
+constexpr int kLightPairs = 256;
+constexpr double kLightMean = 48.0;
+constexpr size_t kLightLds = 40 * 1024;  // four workgroups of four waves per CU
+
+// The light kernel of P's mode and rounding order (nullptr: none).
+static const void* light_kernel(const PairParams& P, int batch)
+{
+#define CF_K(M, F, B)                                                                                          \
+    if (P.mode == M && P.r2form == F && batch == B) return (const void*)&k_pairs_light<M, F, B>;
+    CF_K(MODE_DD, R2_SUM_XY_Z, 0) CF_K(MODE_DD, R2_FMA_DZ_DY_DX, 0)
+    CF_K(MODE_XI, R2_SUM_XY_Z, 0) CF_K(MODE_XI, R2_X_SUM_YZ, 0) CF_K(MODE_XI, R2_FMA_DZ_DY_DX, 0)
+    CF_K(MODE_RPPI, RP_SUM, 0) CF_K(MODE_RPPI, RP_FMA, 0) CF_K(MODE_WP, RP_SUM, 0) CF_K(MODE_WP, RP_FMA, 0)
+    CF_K(MODE_SMU, R2_SUM_XY_Z, 0) CF_K(MODE_SMU, R2_FMA_DX_DY_DZ, 0)
+    CF_K(MODE_RPPI_MOCKS, R2_SUM_XY_Z, 0) CF_K(MODE_SMU_MOCKS, R2_SUM_XY_Z, 0)
+    CF_K(MODE_DD, R2_SUM_XY_Z, 1) CF_K(MODE_DD, R2_FMA_DZ_DY_DX, 1)
+#undef CF_K
+    return nullptr;
+}
+
+// Launches k_pairs_light with an LDS histogram of P's slots (`copies` of it, set
+// so that four workgroups fit a CU). Returns 0 without launching when one copy
+// does not fit.
+static int launch_light(int ncp, const CellPairRec* cps, const DevLattice* lats, int batch, const PairParams& P0,
+                        const double* d_edges, const unsigned short* d_lut, unsigned long long* g_np, double* g_avg,
+                        double* g_w, bool dry)
+{
+    Engine& E = eng();
+    PairParams P = P0;
+    const size_t per_slot = 8 + (P.need_avg ? 8 : 0) + (P.need_w ? 8 : 0);
+    const size_t fixed = (size_t)P.nbin * 8 + (size_t)((P.lut_n + 1) & ~1) * 2;
+    auto lds_for = [&](int r) { return (size_t)(batch ? 4 : 1) * P.nslots * per_slot * r + fixed; };
+    const void* kfn = light_kernel(P, batch);
+    const size_t cap = std::min(kLightLds, E.lds_max);
+    if (!kfn || lds_for(1) > cap) return 0;
+    if (dry) return 1;
+    int R = 1;
+    while (R < 32 && lds_for(2 * R) <= cap) R *= 2;
+    P.hist_copies = R;
+    const long waves = (long)E.ncu * 16;
+    // about four chunks a wave, in a batch long ones (a change of catalog flushes)
+    int light = kLightPairs;
+    int chunk = (int)std::min<long>(batch ? 1024 : 256, std::max<long>(64, ((long)ncp / (4 * waves)) & ~63l));
+    const long need = ((long)ncp + 4 * chunk - 1) / (4 * chunk);
+    const unsigned blocks = (unsigned)std::max<long>(1, std::min<long>(need, waves / 4));
+    void* kargs[] = {&P, &lats, &cps, &ncp, &light, &chunk, &d_edges, &d_lut, &g_np, &g_avg, &g_w};
+    CF_CHECK(hipLaunchKernel(kfn, dim3(blocks), dim3(256), kargs, lds_for(R), E.stream));
+    CF_CHECK(hipGetLastError());
+    return 1;
+}
+
 static int tuned_shape(int batch, PairParams& P, int nslots, int nbin, TunedShape& out)
 {
     Engine& E = eng();
@@ -1112,7 +1163,7 @@ static int tuned_shape(int batch, PairParams& P, int nslots, int nbin, TunedShap
 // appended to the cost model's samples when recording is on).
 static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats, int batch, PairParams& P, int nslots,
                         int nbin, const double* d_edges, const unsigned short* d_lut, unsigned long long* g_np,
-                        double* g_avg, double* g_w, bool timed, TunedRun& T)
+                        double* g_avg, double* g_w, bool timed, double tested, TunedRun& T)
 {
     Engine& E = eng();
     TunedShape ts;
@@ -1124,6 +1175,11 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
     const size_t lds = ts.lds;
     const int per_cu = ts.per_cu;
     const long max_blocks = (long)E.ncu * per_cu;
+    // (per-cell-pair timings need every cell pair in the list)
+    const int light = !gh && !timed && P.dense_mode == 0 && tested <= kLightMean * ncp &&
+                              launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, true)
+                          ? kLightPairs
+                          : 0;
 
     // ---- cost prediction and order
     CF_CHECK(hipEventRecord(E.ev_list, E.stream));
@@ -1149,7 +1205,7 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
         CF_CHECK(hipGetLastError());
         total = (double*)E.arena.get("s_total", sizeof(double));
         k_fill_u64<<<1, 64, 0, E.stream>>>(1, (unsigned long long*)total, 0ull);  // +0.0
-        k_cost_total<<<std::min(nb, 1024), 256, 0, E.stream>>>(ncp, cost, total);
+        k_cost_total<<<std::min(nb, 256), 256, 0, E.stream>>>(ncp, cost, total);
         const int nsb = (ncp + kSortBlock - 1) / kSortBlock;
         const int64_t nmat = (int64_t)kSortBuckets * nsb;
         int* bcount = (int*)E.arena.get("s_bcount", sizeof(int) * (size_t)(nmat + 1));
@@ -1173,14 +1229,16 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
     const double split = sp ? atof(sp) : (double)kSplitPerWave;
     // split <= 0: no splitting (cap = total)
     const double cap_div = split > 0 ? (double)max_blocks * nwaves * split : 1.0;
-    k_count_chunks<<<nb, 256, 0, E.stream>>>(ncp, order, cps, lats, batch, cost, total, cap_div, nparts, nch);
+    k_count_chunks<<<nb, 256, 0, E.stream>>>(ncp, order, cps, lats, batch, cost, total, cap_div, nparts, nch,
+                                             nullptr, light);
     CF_CHECK(hipGetLastError());
     device_scan(nch, off, ncp, "wi_scan");
     int nitems = 0;
     CF_CHECK(hipMemcpyAsync(&nitems, off + ncp, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     CF_CHECK(hipStreamSynchronize(E.stream));
     WorkItem* items = (WorkItem*)E.arena.get("wi_items", sizeof(WorkItem) * ((size_t)nitems + 1));
-    k_emit_chunks<<<nb, 256, 0, E.stream>>>(ncp, order, cps, lats, batch, P, off, nparts, items);
+    k_emit_chunks<<<nb, 256, 0, E.stream>>>(ncp, order, cps, lats, batch, P, off, nparts, items,
+                                            nullptr, INT_MAX, light);
     CF_CHECK(hipGetLastError());
     int* counter = (int*)E.arena.get("wi_counter", sizeof(int) * kQueues * kCounterStride);
     k_fill_i32<<<1, 256, 0, E.stream>>>(kQueues * kCounterStride, counter, 0);
@@ -1218,7 +1276,9 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
 
     void* kargs[] = {&P, &lats, &cps, &items, &d_nitems, &counter, &d_edges, &d_lut, &g_np, &g_avg, &g_w, &ticks, &cu, &single};
     CF_CHECK(hipEventRecord(E.ev0, E.stream));
-    CF_CHECK(hipLaunchKernel(kfn, dim3((unsigned)blocks), dim3(threads), kargs, lds, E.stream));
+    if (light) launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, false);
+    if (!light || nitems > 0)
+        CF_CHECK(hipLaunchKernel(kfn, dim3((unsigned)blocks), dim3(threads), kargs, lds, E.stream));
     CF_CHECK(hipGetLastError());
     CF_CHECK(hipEventRecord(E.ev1, E.stream));
     if (record) {
@@ -1592,7 +1652,7 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     bool tuned = ncp > 0 && E.engine_kind != CF_AMD_ENGINE_PLAIN;
     if (tuned) {
         const int rc = launch_tuned(ncp, cps, lats_for(L1, L2), 0, P, (int)nslots, nbin, d_edges, d_lut, g_np,
-                                    g_avg, g_w, c.cell_timer || E.model.recording, T);
+                                    g_avg, g_w, c.cell_timer || E.model.recording, tested, T);
         if (rc == kNoTunedFit) {
             // more edges than a workgroup's LDS holds next to the queues: plain kernel
             tuned = false;
@@ -1627,7 +1687,7 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     if (need_w) {
         double* ws = (double*)E.arena.get("wsums", sizeof(double) * 2);
         fill_u64(ws, 2);
-        if (c.N1 > 0) k_weight_sums<<<256, 256, 0, E.stream>>>(c.N1, L1.d4, ws);
+        if (c.N1 > 0) k_weight_sums<<<weight_blocks(c.N1), 256, 0, E.stream>>>(c.N1, L1.d4, ws);
         CF_CHECK(hipGetLastError());
         double h[2];
         CF_CHECK(hipMemcpyAsync(h, ws, sizeof h, hipMemcpyDeviceToHost, E.stream));
@@ -1870,7 +1930,7 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
     TunedRun T;
     if (ncp_all > 0) {
         const int rc = launch_tuned(ncp_all, cps, lats, 1, P, nslots, nbin, d_edges, d_lut, g_np, g_avg, g_w,
-                                    E.model.recording, T);
+                                    E.model.recording, tested_all, T);
         if (rc == kNoTunedFit) {
             fprintf(stderr, "Error: %d bins are more than the batched kernel's LDS holds; count the catalogs with "
                             "countpairs one at a time\n", nbin - 1);
@@ -1893,7 +1953,7 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         double* ws = (double*)E.arena.get("bwsums", sizeof(double) * 2 * ncat);
         fill_u64(ws, 2 * (int64_t)ncat);
         for (int k = 0; k < ncat; k++)
-            if (ND[k] > 0) k_weight_sums<<<64, 256, 0, E.stream>>>(ND[k], hl[k].d4, ws + 2 * k);
+            if (ND[k] > 0) k_weight_sums<<<weight_blocks(ND[k]), 256, 0, E.stream>>>(ND[k], hl[k].d4, ws + 2 * k);
         CF_CHECK(hipGetLastError());
         CF_CHECK(hipMemcpyAsync(wsums.data(), ws, sizeof(double) * 2 * ncat, hipMemcpyDeviceToHost, E.stream));
     }
@@ -1999,9 +2059,6 @@ struct GraphScan {
         if (nblocks > 1) {
             run(lv[level].first, lv[level].second, nblocks, st, level + 1);
             k_scan_add<<<(unsigned)nblocks, kScanBlock, 0, st>>>(n, out, lv[level].second);
-            k_copy_int<<<1, 64, 0, st>>>(lv[level].second + nblocks, out + n);
-        } else {
-            k_copy_int<<<1, 64, 0, st>>>(lv[level].first, out + n);
         }
     }
 };
@@ -2273,7 +2330,7 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         k_bg_cp_offset<<<1, 64, 0, st>>>(k, pos, cand_cap, G.cp_off, G.pairs_cap, G.fail);
         k_bg_cellpair_emit<<<(unsigned)std::min<int64_t>((cand_cap + 255) / 256, 1024), 256, 0, st>>>(
             ck, cand_cap, tmpl[k].bstart, tmpl[k].bounds, pos, G.cp_off, k, G.pairs_cap, cps, G.tested);
-        if (need_w && n > 0) k_weight_sums<<<64, 256, 0, st>>>(n, tmpl[k].d4, G.ws + 2 * k);
+        if (need_w && n > 0) k_weight_sums<<<weight_blocks(n), 256, 0, st>>>(n, tmpl[k].d4, G.ws + 2 * k);
     }
     k_oob_flag<<<1, 64, 0, st>>>(oob, G.fail, kBgFailOob);
     // work list as launch_tuned builds it (cost order, heavy cell pairs first
@@ -2289,7 +2346,7 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
             k_cost_heuristic<<<pblk, 256, 0, st>>>(G.pairs_cap, cps, lats, 1, cost, ncp_dev);
         }
         fill_z(total, 1);
-        k_cost_total<<<std::min<unsigned>(pblk, 1024), 256, 0, st>>>(G.pairs_cap, cost, total, ncp_dev);
+        k_cost_total<<<std::min<unsigned>(pblk, 256), 256, 0, st>>>(G.pairs_cap, cost, total, ncp_dev);
         k_cost_hist<<<(unsigned)nsb, 256, 0, st>>>(G.pairs_cap, cost, total, heavy, (int)nsb, bcount, ncp_dev);
         scan.run(bcount, boff, nmat, st);
         k_cost_place<<<(unsigned)nsb, 256, 0, st>>>(G.pairs_cap, cost, total, heavy, (int)nsb, boff, order,

@@ -156,7 +156,8 @@ __global__ void k_index_scatter(int64_t n, const int* __restrict__ bucket, const
     if (b >= 0) idx[bstart[b] + rank[i]] = (int)i;  // b < 0: outside the grid, reported by the host
 }
 
-// Exclusive scan over int32 counts, three phases, 1024 items per block.
+// Exclusive scan over int32 counts, three phases, 1024 items per block; the
+// total goes to out[n] (written by the kernels: a copy of 4 bytes costs a launch).
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 4;
 
@@ -195,7 +196,10 @@ __global__ void k_scan_blocks(int64_t n, const int* __restrict__ in, int* __rest
         if (base + k < n) out[base + k] = ex;
         ex += v[k];
     }
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
+    if (threadIdx.x == 0) {
+        block_sums[blockIdx.x] = tot;
+        if (gridDim.x == 1) out[n] = tot;
+    }
 }
 
 __global__ void k_scan_add(int64_t n, int* __restrict__ out, const int* __restrict__ block_offsets)
@@ -204,6 +208,7 @@ __global__ void k_scan_add(int64_t n, int* __restrict__ out, const int* __restri
     const int add = block_offsets[blockIdx.x];
     for (int k = 0; k < kScanItems; k++)
         if (base + k < n) out[base + k] += add;
+    if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) out[n] = block_offsets[gridDim.x];
 }
 
 // Position of (x, y, z), b bits each, on the 3-D Hilbert curve (J. Skilling,
@@ -424,7 +429,8 @@ __global__ __launch_bounds__(kBigThreads) void k_build_big(const T* X, const T* 
     build_big(X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, big);
 }
 
-// Sums of the weights and of their squares over the grid-ordered records.
+// Sums of the weights and of their squares over the grid-ordered records
+// (workgroups of 256).
 __global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double* __restrict__ out)
 {
     double s = 0, s2 = 0;
@@ -437,9 +443,16 @@ __global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double*
         s += __shfl_xor(s, o, 64);
         s2 += __shfl_xor(s2, o, 64);
     }
+    // one atomic per workgroup and sum (they are serialized, ~14 ns each)
+    __shared__ double part[2][4];
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&out[0], s);
-        atomicAdd(&out[1], s2);
+        part[0][threadIdx.x >> 6] = s;
+        part[1][threadIdx.x >> 6] = s2;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const double* p = part[threadIdx.x];
+        atomicAdd(&out[threadIdx.x], (p[0] + p[1]) + (p[2] + p[3]));
     }
 }
 
@@ -569,8 +582,9 @@ __global__ void k_cellpair_flag(NgbArgs a, int64_t ncells, int nngb, const int* 
 // workgroup, as every atomic on the single counter is serialized.
 __global__ void k_cellpair_emit(NgbArgs a, int64_t ncells, int nngb, const int* __restrict__ bs1,
                                 const int* __restrict__ bs2, const double* __restrict__ bd1,
-                                const double* __restrict__ bd2, const int* __restrict__ pos,
-                                CellPairRec* __restrict__ out, double* __restrict__ tested, int cat)
+                                const double* __restrict__ bd2, const int* __restrict__ flags,
+                                const int* __restrict__ pos, CellPairRec* __restrict__ out,
+                                double* __restrict__ tested, int cat)
 {
     __shared__ double part[4];
     const int64_t total = ncells * nngb;
@@ -578,7 +592,8 @@ __global__ void k_cellpair_emit(NgbArgs a, int64_t ncells, int nngb, const int* 
     for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
          t += (int64_t)gridDim.x * blockDim.x) {
         CellPairRec r = {};
-        if (neighbour_added(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r)) {
+        // (a kept candidate only needs its record again, not the duplicate check)
+        if (flags[t] && eval_neighbour(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r)) {
             r.pad = cat;
             out[pos[t]] = r;
             const double n1 = (double)cell_count(bs1, r.c1), n2 = (double)cell_count(bs2, r.c2);
@@ -1063,8 +1078,9 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T* fresh_k(co
 
 // Decides one (i, j) pair in FP64 exactly as the reference does and adds it to
 // the LDS histogram. (xpos, ypos, zpos) = primary position plus the cell pair's
-// wrap; (xj, yj, zj) = secondary position. `ok` masks lanes without a pair.
-template <int MODE, int R2F, bool GH, int FL>
+// wrap; (xj, yj, zj) = secondary position. `ok` masks lanes without a pair. UNI:
+// cpp and l1p are the same in all lanes.
+template <int MODE, int R2F, bool GH, int FL, bool UNI = true>
 __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRec* cpp, const DevLattice* l1p, int i,
                                            int ok, double xpos, double ypos, double zpos, double wi, double xj,
                                            double yj, double zj, double wj, KernelLds& S)
@@ -1107,8 +1123,8 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
         }
         // pruning replay for pairs near the 3-D limit (the 3-D kernels' rules)
         if (sep2<R2F>(dx, dy, dz) >= P.near_lo2) {
-            const CellPairRec* c = fresh(cpp);
-            const DevLattice* l1 = fresh(l1p);
+            const CellPairRec* c = UNI ? fresh(cpp) : cpp;
+            const DevLattice* l1 = UNI ? fresh(l1p) : l1p;
             ITerms t = {};
             const double4 p = l1->d4[i];
             i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
@@ -1133,8 +1149,8 @@ __device__ __forceinline__ void exact_pair(const PairParams& P, const CellPairRe
     const bool near = r2 >= P.near_lo2 || (MODE != MODE_DD && MODE != MODE_XI && adz >= P.near_lodz);
     if (near) {
         // the cell pair record and the primary set, loaded here
-        const CellPairRec* c = fresh(cpp);
-        const DevLattice* l1 = fresh(l1p);
+        const CellPairRec* c = UNI ? fresh(cpp) : cpp;
+        const DevLattice* l1 = UNI ? fresh(l1p) : l1p;
         ITerms t = {};
         const double4 p = l1->d4[i];
         i_terms(P, MODE, *c, p.x, p.y, p.z, &t);
@@ -1919,6 +1935,124 @@ CF_TUNED_INST(MODE_DD, R2_FMA_DZ_DY_DX, true)
 #undef CF_TUNED_INST_FL
 #undef CF_TUNED_INST0
 
+// Light cell pairs (at most `light` tests each): one lane per cell pair, which
+// tests its few pairs in FP64 one after the other; the work list of the persistent
+// kernel leaves them out. On sparse grids (a few particles per cell) an item of that
+// kernel is one cell pair: a queue atomic and a chain of dependent loads, some
+// microseconds a wave, for a handful of tests. Wave w takes the chunks w, w + W, ...
+// of `chunk` consecutive cell pairs (a multiple of 64); batched, each wave keeps the
+// histogram of the catalog it is working on.
+template <int MODE, int R2F, bool BATCH>
+__global__ __launch_bounds__(256) void k_pairs_light(PairParams P, const DevLattice* __restrict__ lats,
+                                                     const CellPairRec* __restrict__ cps, int ncp, int light,
+                                                     int chunk, const double* __restrict__ rupp_sqr,
+                                                     const unsigned short* __restrict__ lut_g,
+                                                     unsigned long long* __restrict__ g_np,
+                                                     double* __restrict__ g_avg, double* __restrict__ g_w)
+{
+    extern __shared__ unsigned long long smem_u64[];
+    KernelLds S;
+    const int R = P.hist_copies, nwaves = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    const int nrep = P.nslots * R, nreg = BATCH ? nrep * nwaves : nrep;
+    double* avg0 = reinterpret_cast<double*>(smem_u64 + nreg);
+    double* w0 = avg0 + (P.need_avg ? nreg : 0);
+    double* e = w0 + (P.need_w ? nreg : 0);
+    unsigned short* lut = reinterpret_cast<unsigned short*>(e + P.nbin);
+    const int roff = BATCH ? wave * nrep : 0;
+    S.np = smem_u64 + roff;
+    S.avg = avg0 + roff;
+    S.w = w0 + roff;
+    S.rshift = __builtin_ctz(R);
+    S.lane_copy = lane & (R - 1);
+    S.e = e;
+    S.lut = lut;
+    for (int s = threadIdx.x; s < P.nbin; s += blockDim.x) e[s] = rupp_sqr[s];
+    for (int s = threadIdx.x; s < P.lut_n; s += blockDim.x) lut[s] = lut_g[s];
+    for (int s = threadIdx.x; s < nreg; s += blockDim.x) {
+        smem_u64[s] = 0;
+        if (P.need_avg) avg0[s] = 0;
+        if (P.need_w) w0[s] = 0;
+    }
+    __syncthreads();
+    int cur = -1;
+    const int64_t step = (int64_t)gridDim.x * nwaves * chunk;
+    for (int64_t c0 = ((int64_t)blockIdx.x * nwaves + wave) * chunk; c0 < ncp; c0 += step) {
+        const int64_t c1 = min(c0 + chunk, (int64_t)ncp);
+        for (int64_t t0 = c0; t0 < c1; t0 += 64) {
+            const int64_t t = t0 + lane;
+            const CellPairRec* cpp = cps + (t < c1 ? t : c0);
+            const CellPairRec cp = *cpp;
+            const int cat = BATCH ? cp.pad : 0;
+            const DevLattice* l1p = lats + cat;
+            const DevLattice* l2p = lats + (BATCH ? cat : 1);
+            int s1 = 0, e1 = 0, s2 = 0, e2 = 0;
+            if (t < c1) {
+                s1 = l1p->bstart[cp.c1];
+                e1 = l1p->bstart[cp.c1 + 1];
+                s2 = l2p->bstart[cp.c2];
+                e2 = l2p->bstart[cp.c2 + 1];
+            }
+            if ((int64_t)(e1 - s1) * (e2 - s2) > light) e1 = s1;
+            const double wx = cp.wx * P.xwrap, wy = cp.wy * P.ywrap, wz = cp.wz * P.zwrap;
+            const double4 *d1 = l1p->d4, *d2 = l2p->d4;
+            unsigned long long todo = __ballot(e1 > s1);
+            while (todo) {
+                // the lanes of one catalog at a time
+                int k = 0;
+                unsigned long long mine = todo;
+                if (BATCH) {
+                    k = __builtin_amdgcn_readlane(cat, __builtin_ctzll(todo));
+                    mine = todo & __ballot(cat == k);
+                    if (k != cur) {
+                        if (cur >= 0) {
+                            __builtin_amdgcn_wave_barrier();
+                            flush_region(P, S, R, (int64_t)cur * P.nslots, lane, 64, g_np, g_avg, g_w);
+                            __builtin_amdgcn_wave_barrier();
+                        }
+                        cur = k;
+                    }
+                }
+                todo &= ~mine;
+                if ((mine >> lane) & 1ull) {
+                    int i = s1, j = cp.same ? s1 + 1 : s2;
+                    double4 pi = d1[i];
+                    pi.x += wx;
+                    pi.y += wy;
+                    pi.z += wz;
+                    while (i < e1) {
+                        if (j < e2) {
+                            const double4 pj = d2[j];
+                            exact_pair<MODE, R2F, false, kFlRuntime, false>(P, cpp, l1p, i, 1, pi.x, pi.y, pi.z, pi.w,
+                                                                            pj.x, pj.y, pj.z, pj.w, S);
+                            j++;
+                        }
+                        if (j >= e2) {
+                            i++;
+                            j = cp.same ? i + 1 : s2;
+                            if (i < e1) {
+                                pi = d1[i];
+                                pi.x += wx;
+                                pi.y += wy;
+                                pi.z += wz;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (BATCH) {
+        if (cur >= 0) {
+            __builtin_amdgcn_wave_barrier();
+            flush_region(P, S, R, (int64_t)cur * P.nslots, lane, 64, g_np, g_avg, g_w);
+        }
+        return;
+    }
+    __syncthreads();
+    flush_region(P, S, R, 0, threadIdx.x, blockDim.x, g_np, g_avg, g_w);
+}
+
 // Largest squared separation between the bounding boxes of a cell pair
 // (primary box shifted by the wrap), per the geometry of the mode, and whether
 // the pair takes the dense path: every pair of its particles is inside the range,
@@ -1960,7 +2094,7 @@ __device__ __forceinline__ float sane_cost(float c)
 __global__ void k_count_chunks(int ncp, const int* __restrict__ order, const CellPairRec* __restrict__ cps,
                                const DevLattice* __restrict__ lats, int batch, const float* __restrict__ cost,
                                const double* __restrict__ total, double cap_div, int* __restrict__ nparts,
-                               int* __restrict__ nitems, const int* __restrict__ ncp_dev = nullptr)
+                               int* __restrict__ nitems, const int* __restrict__ ncp_dev = nullptr, int light = 0)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ncp) return;
@@ -1972,6 +2106,14 @@ __global__ void k_count_chunks(int ncp, const int* __restrict__ order, const Cel
     const int* bs1 = lats[batch ? cps[c].pad : 0].bstart;
     const int n = (int)cell_count(bs1, cps[c].c1);
     const int nch = (n + 63) / 64;
+    if (light > 0) {
+        // k_pairs_light's share
+        const int n2 = (int)cell_count(lats[batch ? cps[c].pad : 1].bstart, cps[c].c2);
+        if ((int64_t)n * n2 <= light) {
+            nitems[t] = 0;
+            return;
+        }
+    }
     int parts = 1;
     if (cost && nch > 0) {
         const double cap = *total / cap_div;
@@ -1987,10 +2129,11 @@ __global__ void k_emit_chunks(int ncp, const int* __restrict__ order, const Cell
                               const DevLattice* __restrict__ lats, int batch, PairParams P,
                               const int* __restrict__ off, const int* __restrict__ nparts,
                               WorkItem* __restrict__ items, const int* __restrict__ ncp_dev = nullptr,
-                              int items_cap = INT_MAX)
+                              int items_cap = INT_MAX, int light = 0)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ncp || (ncp_dev && t >= *ncp_dev)) return;
+    if (light > 0 && off[t + 1] == off[t]) return;
     const int c = order ? order[t] : t;
     const CellPairRec cp = cps[c];
     const int* bs1 = lats[batch ? cp.pad : 0].bstart;

@@ -116,7 +116,14 @@ __global__ void k_cost_total(int ncp, const float* __restrict__ cost, double* __
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < ncp; t += gridDim.x * blockDim.x)
         v += exp2((double)sane_cost(cost[t]));
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0 && v != 0.0) atomicAdd(total, v);
+    // one atomic per workgroup (they are serialized, ~14 ns each)
+    __shared__ double part[4];
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double s = (part[0] + part[1]) + (part[2] + part[3]);
+        if (s != 0.0) atomicAdd(total, s);
+    }
 }
 
 __device__ __forceinline__ float light_threshold(int ncp, const double* total, float heavy)
