@@ -32,6 +32,7 @@
 #include "cf_sched.hip"
 #include "cf_model.hip"
 #include "cf_bgraph.hip"
+#include "cf_batch.hip"
 #include "../../include/corrfunc_theory.h"
 #include "../../include/corrfunc_amd.h"
 #include "../../include/corrfunc_mocks.h"
@@ -429,6 +430,11 @@ static int make_grid(GridSpec& g, const double ext[6], const double gsz[3], cons
     return EXIT_SUCCESS;
 }
 
+// Quanta per unit length of a grid's quantized positions: kQMax quanta cover the
+// largest cell side plus the pair reach, so every position within reach of a cell
+// has an unclamped quantized offset.
+static double grid_qinv(const GridSpec& g) { return (double)kQMax / (fmax(g.xbs, fmax(g.ybs, g.zbs)) + g.qreach); }
+
 // Device counting sort of one particle set into the grid (gridlink_impl.c.src:65-436).
 // Counting-sort gridding launched on the stream without waiting: particles
 // outside the grid are counted into *oob (zeroed by the caller) and skipped.
@@ -456,9 +462,7 @@ static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n,
     int* big = (int*)E.arena.get(tag + "_big", sizeof(int) * (nbig + 1));
     L.bstart = (int*)E.arena.get(tag + "_bstart", sizeof(int) * (nb + 1));
     L.d4 = (double4*)E.arena.get(tag + "_d4", sizeof(double4) * (n + kQPad));
-    // quantum: kQMax quanta cover the largest cell side plus the pair reach, so
-    // every position within reach of a cell has an unclamped quantized offset
-    L.qinv = (double)kQMax / (fmax(g.xbs, fmax(g.ybs, g.zbs)) + g.qreach);
+    L.qinv = grid_qinv(g);
     L.q = (uint2*)E.arena.get(tag + "_q", sizeof(uint2) * (n + kQPad));
     L.bounds = (double*)E.arena.get(tag + "_bounds", sizeof(double) * 6 * L.ncells);
     L.gbox = (double*)E.arena.get(tag + "_gbox", sizeof(double) * 6 * (n / kGroup + L.ncells + 1));
@@ -544,22 +548,29 @@ struct CpPlan {
     DevLattice L1, L2;
 };
 
+static void cellpairs_args(int nx, int ny, int nz, const int refine[3], const int per[3], const double wrap[3],
+                           double max3, double max2, double max1, int min_sep_opt, int autocorr, NgbArgs& a,
+                           int& nngb)
+{
+    a.nx = nx; a.ny = ny; a.nz = nz;
+    a.rx = refine[0]; a.ry = refine[1]; a.rz = refine[2];
+    a.px = per[0]; a.py = per[1]; a.pz = per[2];
+    a.autocorr = autocorr;
+    a.min_sep_opt = min_sep_opt;
+    a.dupcheck = (per[0] || per[1] || per[2]) &&
+                 (nx < 2 * refine[0] + 1 || ny < 2 * refine[1] + 1 || nz < 2 * refine[2] + 1);
+    a.xwrap = wrap[0]; a.ywrap = wrap[1]; a.zwrap = wrap[2];
+    a.max3 = max3; a.max2 = max2; a.max1 = max1;
+    nngb = (2 * refine[0] + 1) * (2 * refine[1] + 1) * (2 * refine[2] + 1);
+}
+
 static int cellpairs_flag(const DevLattice& L1, const DevLattice& L2, const int refine[3], const int per[3],
                           const double wrap[3], double max3, double max2, double max1, int min_sep_opt, int autocorr,
                           CpPlan& cp)
 {
     Engine& E = eng();
     NgbArgs& a = cp.a;
-    a.nx = L1.nx; a.ny = L1.ny; a.nz = L1.nz;
-    a.rx = refine[0]; a.ry = refine[1]; a.rz = refine[2];
-    a.px = per[0]; a.py = per[1]; a.pz = per[2];
-    a.autocorr = autocorr;
-    a.min_sep_opt = min_sep_opt;
-    a.dupcheck = (per[0] || per[1] || per[2]) &&
-                 (L1.nx < 2 * refine[0] + 1 || L1.ny < 2 * refine[1] + 1 || L1.nz < 2 * refine[2] + 1);
-    a.xwrap = wrap[0]; a.ywrap = wrap[1]; a.zwrap = wrap[2];
-    a.max3 = max3; a.max2 = max2; a.max1 = max1;
-    cp.nngb = (2 * refine[0] + 1) * (2 * refine[1] + 1) * (2 * refine[2] + 1);
+    cellpairs_args(L1.nx, L1.ny, L1.nz, refine, per, wrap, max3, max2, max1, min_sep_opt, autocorr, a, cp.nngb);
     cp.total = L1.ncells * cp.nngb;
     cp.L1 = L1;
     cp.L2 = L2;
@@ -1739,6 +1750,115 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
 // DD(r) auto-correlations of many independent catalogs in one device work list
 // and one persistent pair-kernel launch. Catalog k gets exactly the results that
 // countpairs() gives for it with a copy of `options`.
+// Gridding and cell pairs of a whole batch in concatenated arrays (cf_batch.hip).
+// `sets` (ncat + 1 entries, inputs, extents' block numbers and grids filled in)
+// gets its offsets here; fills hl, the work list, its length and the pairs tested.
+static int batch_grid(int ncat, std::vector<BatchSet>& sets, size_t esize, std::vector<DevLattice>& hl,
+                      CellPairRec** cps_out, int* ncp_out, double* tested)
+{
+    Engine& E = eng();
+    BatchSet end = {};
+    for (int k = 0; k < ncat; k++) {
+        BatchSet& s = sets[k];
+        s.p0 = end.p0;
+        s.c0 = end.c0;
+        s.t0 = end.t0;
+        s.pb0 = end.pb0;
+        s.cb0 = end.cb0;
+        s.tb0 = end.tb0;
+        end.p0 += s.n;
+        end.c0 += s.ncells;
+        end.t0 += s.ncand;
+        end.pb0 += (int)((s.n + 255) / 256);
+        end.cb0 += (int)((s.ncells + 3) / 4);
+        end.tb0 += (int)((s.ncand + kEmitItems - 1) / kEmitItems);
+    }
+    end.mb0 = sets[ncat].mb0;
+    sets[ncat] = end;
+    const int64_t N = end.p0, C = end.c0, T = end.t0;
+    BatchSet* d_sets = (BatchSet*)E.arena.get("ba_sets", sizeof(BatchSet) * (size_t)(ncat + 1));
+    CF_CHECK(hipMemcpyAsync(d_sets, sets.data(), sizeof(BatchSet) * (size_t)(ncat + 1), hipMemcpyHostToDevice, E.stream));
+    int* counts = (int*)E.arena.get("ba_cnt", sizeof(int) * (C + 1));
+    int* bucket = (int*)E.arena.get("ba_bucket", sizeof(int) * (N + 1));
+    int* rank = (int*)E.arena.get("ba_rank", sizeof(int) * (N + 1));
+    int* idx = (int*)E.arena.get("ba_idx", sizeof(int) * (N + 1));
+    const int64_t nbig = N / kSmallCell;
+    int* big = (int*)E.arena.get("ba_big", sizeof(int) * (nbig + 1));
+    int* bstart = (int*)E.arena.get("ba_bstart", sizeof(int) * (C + 1));
+    double4* d4 = (double4*)E.arena.get("ba_d4", sizeof(double4) * (N + kQPad));
+    uint2* q = (uint2*)E.arena.get("ba_q", sizeof(uint2) * (N + kQPad));
+    double* bounds = (double*)E.arena.get("ba_bounds", sizeof(double) * 6 * C);
+    double* gbox = (double*)E.arena.get("ba_gbox", sizeof(double) * 6 * (N / kGroup + C + 1));
+    int* flags = (int*)E.arena.get("ba_flags", sizeof(int) * (T + 1));
+    int* pos = (int*)E.arena.get("ba_pos", sizeof(int) * (T + 1));
+    double* d_tested = (double*)E.arena.get("b_tested", sizeof(double) * ncat);
+    unsigned long long* oob = (unsigned long long*)E.arena.get("b_oob", sizeof(unsigned long long));
+    fill_i32(counts, C + 1, 0);
+    fill_i32(big, 1, 0);
+    fill_u64(oob, 1);
+    fill_u64(d_tested, ncat);
+    if (N > 0) {
+        if (esize == 4)
+            kb_bucket_count<float><<<end.pb0, 256, 0, E.stream>>>(d_sets, ncat, bucket, rank, counts, oob);
+        else
+            kb_bucket_count<double><<<end.pb0, 256, 0, E.stream>>>(d_sets, ncat, bucket, rank, counts, oob);
+        CF_CHECK(hipGetLastError());
+    }
+    device_scan(counts, bstart, C, "ba_scan");
+    if (N > 0) kb_index_scatter<<<end.pb0, 256, 0, E.stream>>>(d_sets, ncat, bucket, rank, bstart, idx);
+    const unsigned bb = (unsigned)std::min<int64_t>(nbig, 2 * E.ncu);
+    if (esize == 4) {
+        kb_build_small<float><<<end.cb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, idx, rank, d4, q, bounds, gbox, big);
+        if (bb > 0)
+            kb_build_big<float><<<bb, kBigThreads, 0, E.stream>>>(d_sets, ncat, bstart, idx, rank, d4, q, bounds,
+                                                                  gbox, big);
+    } else {
+        kb_build_small<double><<<end.cb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, idx, rank, d4, q, bounds, gbox,
+                                                              big);
+        if (bb > 0)
+            kb_build_big<double><<<bb, kBigThreads, 0, E.stream>>>(d_sets, ncat, bstart, idx, rank, d4, q, bounds,
+                                                                   gbox, big);
+    }
+    CF_CHECK(hipGetLastError());
+    kb_cellpair_flag<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags);
+    CF_CHECK(hipGetLastError());
+    device_scan(flags, pos, T, "ba_pscan");
+    int ncp = 0;
+    unsigned long long h_oob = 0;
+    CF_CHECK(hipMemcpyAsync(&ncp, pos + T, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    CF_CHECK(hipMemcpyAsync(&h_oob, oob, sizeof h_oob, hipMemcpyDeviceToHost, E.stream));
+    CF_CHECK(hipStreamSynchronize(E.stream));
+    if (check_oob(h_oob) != EXIT_SUCCESS) return EXIT_FAILURE;
+    check_interrupt();
+    CellPairRec* cps = (CellPairRec*)E.arena.get("bcp_all", sizeof(CellPairRec) * ((size_t)ncp + 1));
+    kb_cellpair_emit<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags, pos, cps, d_tested);
+    CF_CHECK(hipGetLastError());
+    std::vector<double> tk(ncat);
+    CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
+    CF_CHECK(hipStreamSynchronize(E.stream));
+    *tested = 0;
+    for (int k = 0; k < ncat; k++) {
+        const BatchSet& s = sets[k];
+        DevLattice& L = hl[k];
+        L.nx = s.g.nx; L.ny = s.g.ny; L.nz = s.g.nz;
+        L.ncells = s.ncells;
+        L.n = s.n;
+        L.xmin = s.g.xmin; L.ymin = s.g.ymin; L.zmin = s.g.zmin;
+        L.xbs = s.g.xbs; L.ybs = s.g.ybs; L.zbs = s.g.zbs;
+        L.xinv = s.g.xinv; L.yinv = s.g.yinv; L.zinv = s.g.zinv;
+        L.qinv = s.g.qinv;
+        L.d4 = d4;
+        L.q = q;
+        L.bstart = bstart + s.c0;
+        L.bounds = bounds + 6 * s.c0;
+        L.gbox = gbox + 6 * s.c0;
+        *tested += tk[k];
+    }
+    *cps_out = cps;
+    *ncp_out = ncp;
+    return EXIT_SUCCESS;
+}
+
 static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, void** W, const char* binfile,
                      struct config_options* options, struct extra_options* extra, std::vector<CallOut>& outs)
 {
@@ -1794,18 +1914,40 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         fprintf(stderr, "boxsize must be specified with periodic wrap.\n");
         return EXIT_FAILURE;
     }
+    std::vector<BatchSet> sets((size_t)ncat + 1, BatchSet{});
     std::vector<double> exts(6 * (size_t)ncat);
     {
         double* d_ext = (double*)E.arena.get("b_ext", sizeof(double) * 6 * ncat);
-        for (int k = 0; k < ncat; k++) device_minmax_async(dx[k], dy[k], dz[k], ND[k], esize, d_ext + 6 * k);
+        int64_t mb = 0;
+        for (int k = 0; k < ncat; k++) {
+            BatchSet& s = sets[k];
+            s.X = dx[k]; s.Y = dy[k]; s.Z = dz[k]; s.W = dw[k];
+            s.n = ND[k];
+            s.mb0 = (int)mb;
+            mb += std::max<int64_t>(1, (ND[k] + kExtentItems - 1) / kExtentItems);
+        }
+        sets[ncat].mb0 = (int)mb;
+        if (mb >= (int64_t)INT32_MAX) {
+            fprintf(stderr, "Error: the batch's particles exceed the engine's indexing\n");
+            return EXIT_FAILURE;
+        }
+        BatchSet* d_sets = (BatchSet*)E.arena.get("ba_sets", sizeof(BatchSet) * (size_t)(ncat + 1));
+        double* part = (double*)E.arena.get("ba_mm", sizeof(double) * 6 * (size_t)mb);
+        CF_CHECK(hipMemcpyAsync(d_sets, sets.data(), sizeof(BatchSet) * (size_t)(ncat + 1), hipMemcpyHostToDevice,
+                                E.stream));
+        if (esize == 4)
+            kb_minmax<float><<<(unsigned)mb, 256, 0, E.stream>>>(d_sets, ncat, part);
+        else
+            kb_minmax<double><<<(unsigned)mb, 256, 0, E.stream>>>(d_sets, ncat, part);
+        kb_minmax_final<<<ncat, 64, 0, E.stream>>>(d_sets, part, d_ext);
+        CF_CHECK(hipGetLastError());
         CF_CHECK(hipMemcpyAsync(exts.data(), d_ext, sizeof(double) * 6 * ncat, hipMemcpyDeviceToHost, E.stream));
         CF_CHECK(hipStreamSynchronize(E.stream));
     }
     std::vector<std::array<int, 3>> refines(ncat), pers(ncat);
     double wrap0[3] = {0, 0, 0}, coord_scale = 0, cs_max = 0, tested_all = 0;
     int rmaxr = 1;
-    unsigned long long* d_oob = (unsigned long long*)E.arena.get("b_oob", sizeof(unsigned long long));
-    fill_u64(d_oob, 1);
+    std::vector<GridSpec> grids(ncat);
     for (int k = 0; k < ncat; k++) {
         struct config_options oc = *options;
         const double* ext = &exts[6 * (size_t)k];
@@ -1841,11 +1983,8 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
             }
         }
         int refine[3];
-        GridSpec g;
+        GridSpec& g = grids[k];
         if (choose_grid(MODE_DD, ND[k], rmax, rmax, 0.0, ext, wrap, &oc, g, refine) != EXIT_SUCCESS)
-            return EXIT_FAILURE;
-        if (gridlink_launch("b" + std::to_string(k), g, ND[k], dx[k], dy[k], dz[k], dw[k], esize, hl[k], d_oob) !=
-            EXIT_SUCCESS)
             return EXIT_FAILURE;
         refines[k] = {refine[0], refine[1], refine[2]};
         pers[k] = {per[0], per[1], per[2]};
@@ -1853,53 +1992,82 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         cs_max = fmax(cs_max, fmax(g.xbs, fmax(g.ybs, g.zbs)));
         for (int d = 0; d < 3; d++) rmaxr = refine[d] > rmaxr ? refine[d] : rmaxr;
     }
-    // cell-pair counts per catalog
-    std::vector<int> ncps(ncat);
-    {
-        int* d_ncp = (int*)E.arena.get("b_ncp", sizeof(int) * ncat);
+    coord_scale = 6 * coord_scale + wrap0[0] + wrap0[1] + wrap0[2] + rmax;
+    // all catalogs in concatenated arrays while these keep to 32-bit indices
+    // (96 catalogs of 2,000-20,000 points: 2,757 launches become 60), else one
+    // catalog after the other
+    int64_t sum_n = 0, sum_cells = 0, sum_cand = 0;
+    for (int k = 0; k < ncat; k++) {
+        BatchSet& s = sets[k];
+        const GridSpec& g = grids[k];
+        s.ncells = (int64_t)g.nx * g.ny * g.nz;
+        cellpairs_args(g.nx, g.ny, g.nz, refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
+                       options->enable_min_sep_opt, 1, s.a, s.nngb);
+        s.ncand = s.ncells * s.nngb;
+        s.g = GridArgs{g.xmin, g.ymin, g.zmin, g.xinv, g.yinv, g.zinv, g.xbs, g.ybs, g.zbs, g.nx, g.ny, g.nz,
+                       grid_qinv(g)};
+        sum_n += s.n;
+        sum_cells += s.ncells;
+        sum_cand += s.ncand;
+    }
+    const bool joint = sum_n < (int64_t)INT32_MAX - 256 && sum_cells < (int64_t)INT32_MAX && sum_cand < (int64_t)1 << 30;
+    CellPairRec* cps = nullptr;
+    int ncp_all = 0;
+    if (joint) {
+        if (batch_grid(ncat, sets, esize, hl, &cps, &ncp_all, &tested_all) != EXIT_SUCCESS) return EXIT_FAILURE;
+    } else {
+        unsigned long long* d_oob = (unsigned long long*)E.arena.get("b_oob", sizeof(unsigned long long));
+        fill_u64(d_oob, 1);
+        for (int k = 0; k < ncat; k++)
+            if (gridlink_launch("b" + std::to_string(k), grids[k], ND[k], dx[k], dy[k], dz[k], dw[k], esize, hl[k],
+                                d_oob) != EXIT_SUCCESS)
+                return EXIT_FAILURE;
+        // cell-pair counts per catalog
+        std::vector<int> ncps(ncat);
+        {
+            int* d_ncp = (int*)E.arena.get("b_ncp", sizeof(int) * ncat);
+            for (int k = 0; k < ncat; k++) {
+                CpPlan cp;
+                if (cellpairs_flag(hl[k], hl[k], refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
+                                   options->enable_min_sep_opt, 1, cp) != EXIT_SUCCESS)
+                    return EXIT_FAILURE;
+                k_copy_int<<<1, 64, 0, E.stream>>>(cp.pos + cp.total, d_ncp + k);
+            }
+            CF_CHECK(hipGetLastError());
+            unsigned long long h_oob = 0;
+            CF_CHECK(hipMemcpyAsync(ncps.data(), d_ncp, sizeof(int) * ncat, hipMemcpyDeviceToHost, E.stream));
+            CF_CHECK(hipMemcpyAsync(&h_oob, d_oob, sizeof(h_oob), hipMemcpyDeviceToHost, E.stream));
+            CF_CHECK(hipStreamSynchronize(E.stream));
+            if (check_oob(h_oob) != EXIT_SUCCESS) return EXIT_FAILURE;
+        }
+        std::vector<int> cp_off(ncat);
         for (int k = 0; k < ncat; k++) {
+            cp_off[k] = ncp_all;
+            if ((int64_t)ncp_all + ncps[k] >= (int64_t)INT32_MAX) {
+                fprintf(stderr, "Error: the batch's cell pairs exceed the engine's 32-bit indexing\n");
+                return EXIT_FAILURE;
+            }
+            ncp_all += ncps[k];
+        }
+        check_interrupt();
+        // concatenated work list, emitted in place
+        cps = (CellPairRec*)E.arena.get("bcp_all", sizeof(CellPairRec) * ((size_t)ncp_all + 1));
+        double* d_tested = (double*)E.arena.get("b_tested", sizeof(double) * ncat);
+        fill_u64(d_tested, ncat);
+        for (int k = 0; k < ncat; k++) {
+            if (ncps[k] == 0) continue;
             CpPlan cp;
             if (cellpairs_flag(hl[k], hl[k], refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
                                options->enable_min_sep_opt, 1, cp) != EXIT_SUCCESS)
                 return EXIT_FAILURE;
-            k_copy_int<<<1, 64, 0, E.stream>>>(cp.pos + cp.total, d_ncp + k);
+            cellpairs_emit(cp, cps + cp_off[k], d_tested + k, k);
         }
-        CF_CHECK(hipGetLastError());
-        unsigned long long h_oob = 0;
-        CF_CHECK(hipMemcpyAsync(ncps.data(), d_ncp, sizeof(int) * ncat, hipMemcpyDeviceToHost, E.stream));
-        CF_CHECK(hipMemcpyAsync(&h_oob, d_oob, sizeof(h_oob), hipMemcpyDeviceToHost, E.stream));
-        CF_CHECK(hipStreamSynchronize(E.stream));
-        if (check_oob(h_oob) != EXIT_SUCCESS) return EXIT_FAILURE;
-    }
-    int ncp_all = 0;
-    std::vector<int> cp_off(ncat);
-    for (int k = 0; k < ncat; k++) {
-        cp_off[k] = ncp_all;
-        if ((int64_t)ncp_all + ncps[k] >= (int64_t)INT32_MAX) {
-            fprintf(stderr, "Error: the batch's cell pairs exceed the engine's 32-bit indexing\n");
-            return EXIT_FAILURE;
+        {
+            std::vector<double> tk(ncat);
+            CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
+            CF_CHECK(hipStreamSynchronize(E.stream));
+            for (int k = 0; k < ncat; k++) tested_all += tk[k];
         }
-        ncp_all += ncps[k];
-    }
-    check_interrupt();
-    coord_scale = 6 * coord_scale + wrap0[0] + wrap0[1] + wrap0[2] + rmax;
-    // concatenated work list, emitted in place
-    CellPairRec* cps = (CellPairRec*)E.arena.get("bcp_all", sizeof(CellPairRec) * ((size_t)ncp_all + 1));
-    double* d_tested = (double*)E.arena.get("b_tested", sizeof(double) * ncat);
-    fill_u64(d_tested, ncat);
-    for (int k = 0; k < ncat; k++) {
-        if (ncps[k] == 0) continue;
-        CpPlan cp;
-        if (cellpairs_flag(hl[k], hl[k], refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
-                           options->enable_min_sep_opt, 1, cp) != EXIT_SUCCESS)
-            return EXIT_FAILURE;
-        cellpairs_emit(cp, cps + cp_off[k], d_tested + k, k);
-    }
-    {
-        std::vector<double> tk(ncat);
-        CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
-        CF_CHECK(hipStreamSynchronize(E.stream));
-        for (int k = 0; k < ncat; k++) tested_all += tk[k];
     }
     const double t_grid = now_s();
 
@@ -1952,8 +2120,12 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
     if (need_w) {
         double* ws = (double*)E.arena.get("bwsums", sizeof(double) * 2 * ncat);
         fill_u64(ws, 2 * (int64_t)ncat);
-        for (int k = 0; k < ncat; k++)
-            if (ND[k] > 0) k_weight_sums<<<weight_blocks(ND[k]), 256, 0, E.stream>>>(ND[k], hl[k].d4, ws + 2 * k);
+        if (joint)
+            kb_weight_sums<<<sets[ncat].mb0, 256, 0, E.stream>>>((const BatchSet*)E.arena.get("ba_sets", 0), ncat,
+                                                                 hl[0].d4, ws);
+        else
+            for (int k = 0; k < ncat; k++)
+                if (ND[k] > 0) k_weight_sums<<<weight_blocks(ND[k]), 256, 0, E.stream>>>(ND[k], hl[k].d4, ws + 2 * k);
         CF_CHECK(hipGetLastError());
         CF_CHECK(hipMemcpyAsync(wsums.data(), ws, sizeof(double) * 2 * ncat, hipMemcpyDeviceToHost, E.stream));
     }

@@ -41,12 +41,15 @@ __device__ __forceinline__ double wave_max_d(double v)
 }
 
 // ------------------------------------------------------------ extent (a2)
+// Extent of the points i, i + step, ... below end, reduced over a workgroup of
+// 256 into out[0..5].
 template <typename T>
-__global__ void k_minmax(int64_t n, const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-                         double* __restrict__ partial)
+__device__ __forceinline__ void minmax_block(int64_t i, int64_t end, int64_t step, const T* __restrict__ X,
+                                             const T* __restrict__ Y, const T* __restrict__ Z,
+                                             double* __restrict__ out)
 {
     double mn[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, mx[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    for (; i < end; i += step) {
         const double v[3] = {(double)X[i], (double)Y[i], (double)Z[i]};
         for (int d = 0; d < 3; d++) { mn[d] = fmin(mn[d], v[d]); mx[d] = fmax(mx[d], v[d]); }
     }
@@ -62,12 +65,20 @@ __global__ void k_minmax(int64_t n, const T* __restrict__ X, const T* __restrict
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        for (int d = 0; d < 6; d++) partial[blockIdx.x * 6 + d] = s[d][0];
+        for (int d = 0; d < 6; d++) out[d] = s[d][0];
+}
+template <typename T>
+__global__ void k_minmax(int64_t n, const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
+                         double* __restrict__ partial)
+{
+    minmax_block(blockIdx.x * (int64_t)blockDim.x + threadIdx.x, n, (int64_t)gridDim.x * blockDim.x, X, Y, Z,
+                 partial + blockIdx.x * 6);
 }
 
 // One wave: the lanes reduce strided subsets of the block partials, then the
 // wave (min/max are exact, so the order does not matter).
-__global__ void k_minmax_final(int nblocks, const double* __restrict__ partial, double* __restrict__ out)
+__device__ __forceinline__ void minmax_reduce(int nblocks, const double* __restrict__ partial,
+                                              double* __restrict__ out)
 {
     const int lane = (int)threadIdx.x;
     double r[6] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX};
@@ -82,6 +93,10 @@ __global__ void k_minmax_final(int nblocks, const double* __restrict__ partial, 
     }
     if (lane == 0)
         for (int d = 0; d < 6; d++) out[d] = r[d];
+}
+__global__ void k_minmax_final(int nblocks, const double* __restrict__ partial, double* __restrict__ out)
+{
+    minmax_reduce(nblocks, partial, out);
 }
 
 // --------------------------------------------------------- gridding (a5)
@@ -431,10 +446,11 @@ __global__ __launch_bounds__(kBigThreads) void k_build_big(const T* X, const T* 
 
 // Sums of the weights and of their squares over the grid-ordered records
 // (workgroups of 256).
-__global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double* __restrict__ out)
+__device__ __forceinline__ void weight_sums_block(int64_t i, int64_t end, int64_t step,
+                                                  const double4* __restrict__ d4, double* __restrict__ out)
 {
     double s = 0, s2 = 0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    for (; i < end; i += step) {
         const double w = d4[i].w;
         s += w;
         s2 += w * w;
@@ -454,6 +470,10 @@ __global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double*
         const double* p = part[threadIdx.x];
         atomicAdd(&out[threadIdx.x], (p[0] + p[1]) + (p[2] + p[3]));
     }
+}
+__global__ void k_weight_sums(int64_t n, const double4* __restrict__ d4, double* __restrict__ out)
+{
+    weight_sums_block(blockIdx.x * (int64_t)blockDim.x + threadIdx.x, n, (int64_t)gridDim.x * blockDim.x, d4, out);
 }
 
 // Device-to-device copy: n16 16-byte words through the vector path (grid-stride),
