@@ -23,7 +23,7 @@ struct BatchSet {
     NgbArgs a;
 };
 constexpr int kExtentItems = 4096;  // particles per block of the extent and weight kernels
-constexpr int kEmitItems = 4096;    // candidates per block of kb_cellpairs
+constexpr int kEmitItems = 4096;    // candidates per block of the cell-pair kernels
 
 // The catalog whose blocks (first one: member F) contain block b; s[ncat].*F is
 // the number of blocks, and a catalog may have none.
@@ -123,28 +123,12 @@ __global__ __launch_bounds__(kBigThreads) void kb_build_big(const BatchSet* __re
     }
 }
 
-__global__ void kb_cellpair_flag(const BatchSet* __restrict__ sets, int ncat, const int* __restrict__ bstart,
-                                 const double* __restrict__ bounds, int* __restrict__ flags)
-{
-    const BatchSet& s = sets[batch_find<&BatchSet::tb0>(sets, ncat, blockIdx.x)];
-    const int* bs = bstart + s.c0;
-    const double* bd = bounds + 6 * s.c0;
-    const int64_t t0 = (int64_t)(blockIdx.x - s.tb0) * kEmitItems, t1 = min(t0 + kEmitItems, s.ncand);
-    for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-        CellPairRec r = {};
-        flags[s.t0 + t] = neighbour_added(s.a, t / s.nngb, (int)(t % s.nngb), bs, bs, bd, bd, &r);
-    }
-}
-
-// The flagged candidates' records at their scan positions; the pairs tested of
-// a catalog are added to tested[catalog].
-__global__ __launch_bounds__(256) void kb_cellpair_emit(const BatchSet* __restrict__ sets, int ncat,
+// The pairs tested of a catalog are added to tested[catalog].
+__global__ __launch_bounds__(256) void kb_cellpair_flag(const BatchSet* __restrict__ sets, int ncat,
                                                         const int* __restrict__ bstart,
-                                                        const double* __restrict__ bounds,
-                                                        const int* __restrict__ flags, const int* __restrict__ pos,
-                                                        CellPairRec* __restrict__ out, double* __restrict__ tested)
+                                                        const double* __restrict__ bounds, int* __restrict__ flags,
+                                                        double* __restrict__ tested)
 {
-    __shared__ double part[4];
     const int k = batch_find<&BatchSet::tb0>(sets, ncat, blockIdx.x);
     const BatchSet& s = sets[k];
     const int* bs = bstart + s.c0;
@@ -153,19 +137,31 @@ __global__ __launch_bounds__(256) void kb_cellpair_emit(const BatchSet* __restri
     double my = 0;
     for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
         CellPairRec r = {};
+        const int f = neighbour_added(s.a, t / s.nngb, (int)(t % s.nngb), bs, bs, bd, bd, &r);
+        flags[s.t0 + t] = f;
+        if (f) my += pair_tests(r, bs, bs);
+    }
+    add_tests(my, &tested[k]);
+}
+
+// The flagged candidates' records at their scan positions.
+__global__ __launch_bounds__(256) void kb_cellpair_emit(const BatchSet* __restrict__ sets, int ncat,
+                                                        const int* __restrict__ bstart,
+                                                        const double* __restrict__ bounds,
+                                                        const int* __restrict__ flags, const int* __restrict__ pos,
+                                                        CellPairRec* __restrict__ out)
+{
+    const int k = batch_find<&BatchSet::tb0>(sets, ncat, blockIdx.x);
+    const BatchSet& s = sets[k];
+    const int* bs = bstart + s.c0;
+    const double* bd = bounds + 6 * s.c0;
+    const int64_t t0 = (int64_t)(blockIdx.x - s.tb0) * kEmitItems, t1 = min(t0 + kEmitItems, s.ncand);
+    for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
+        CellPairRec r = {};
         if (flags[s.t0 + t] && eval_neighbour(s.a, t / s.nngb, (int)(t % s.nngb), bs, bs, bd, bd, &r)) {
             r.pad = k;
             out[pos[s.t0 + t]] = r;
-            const double n1 = (double)cell_count(bs, r.c1), n2 = (double)cell_count(bs, r.c2);
-            my += r.same ? n1 * (n1 - 1) * 0.5 : n1 * n2;
         }
-    }
-    for (int o = 32; o > 0; o >>= 1) my += __shfl_xor(my, o, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = my;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const double v = (part[0] + part[1]) + (part[2] + part[3]);
-        if (v != 0) atomicAdd(&tested[k], v);
     }
 }
 

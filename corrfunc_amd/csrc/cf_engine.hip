@@ -518,27 +518,25 @@ static int check_oob(unsigned long long n_oob)
     return EXIT_SUCCESS;
 }
 
+// Gridding of one set of a call; its count of particles outside the grid stays on
+// the device (*oob) until the call's next synchronisation.
 static int gridlink_device(const std::string& tag, const GridSpec& g, int64_t n, const void* X, const void* Y,
-                           const void* Z, const void* W, size_t esize, DevLattice& L)
+                           const void* Z, const void* W, size_t esize, DevLattice& L, unsigned long long** oob)
 {
     Engine& E = eng();
-    unsigned long long* oob = (unsigned long long*)E.arena.get(tag + "_oob", 8);
-    fill_u64(oob, 1);
-    if (gridlink_launch(tag, g, n, X, Y, Z, W, esize, L, oob) != EXIT_SUCCESS) return EXIT_FAILURE;
-    unsigned long long h_oob = 0;
-    CF_CHECK(hipMemcpyAsync(&h_oob, oob, 8, hipMemcpyDeviceToHost, E.stream));
-    CF_CHECK(hipStreamSynchronize(E.stream));
-    return check_oob(h_oob);
+    *oob = (unsigned long long*)E.arena.get(tag + "_oob", 8);
+    fill_u64(*oob, 1);
+    return gridlink_launch(tag, g, n, X, Y, Z, W, esize, L, *oob);
 }
 
 // Workgroups of k_weight_sums: 8 records a thread, at most 512 (two atomics each).
 static unsigned weight_blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(512, n / 2048)); }
 
 // Device work list of neighbour-cell pairs (gridlink_impl.c.src:439-625), in
-// two steps: cellpairs_flag marks the kept (cell, neighbour) candidates and
-// scans them (the count lands at plan.pos[plan.total] on the device);
-// cellpairs_emit writes the records in the reference's order and adds the pairs
-// tested to *dtested.
+// two steps: cellpairs_flag marks the kept (cell, neighbour) candidates, adds the
+// pairs tested to dtested[0 .. kTestedSlots - 1] and scans the marks (the count
+// lands at plan.pos[plan.total] on the device); cellpairs_emit writes the records
+// in the reference's order.
 struct CpPlan {
     NgbArgs a;
     int nngb = 0;
@@ -566,7 +564,7 @@ static void cellpairs_args(int nx, int ny, int nz, const int refine[3], const in
 
 static int cellpairs_flag(const DevLattice& L1, const DevLattice& L2, const int refine[3], const int per[3],
                           const double wrap[3], double max3, double max2, double max1, int min_sep_opt, int autocorr,
-                          CpPlan& cp)
+                          double* dtested, CpPlan& cp)
 {
     Engine& E = eng();
     NgbArgs& a = cp.a;
@@ -582,38 +580,47 @@ static int cellpairs_flag(const DevLattice& L1, const DevLattice& L2, const int 
     cp.pos = (int*)E.arena.get("cp_pos", sizeof(int) * (cp.total + 1));
     const unsigned blocks = (unsigned)((cp.total + 255) / 256);
     k_cellpair_flag<<<blocks, 256, 0, E.stream>>>(a, L1.ncells, cp.nngb, L1.bstart, L2.bstart, L1.bounds, L2.bounds,
-                                                  cp.flags);
+                                                  cp.flags, dtested);
     CF_CHECK(hipGetLastError());
     device_scan(cp.flags, cp.pos, cp.total, "cp_scan");
     return EXIT_SUCCESS;
 }
 
-static void cellpairs_emit(const CpPlan& cp, CellPairRec* out, double* dtested, int cat)
+static void cellpairs_emit(const CpPlan& cp, CellPairRec* out, int cat)
 {
     Engine& E = eng();
-    const unsigned blocks = (unsigned)std::min<int64_t>((cp.total + 255) / 256, 1024);
+    const unsigned blocks = (unsigned)((cp.total + 255) / 256);
     k_cellpair_emit<<<blocks, 256, 0, E.stream>>>(cp.a, cp.L1.ncells, cp.nngb, cp.L1.bstart, cp.L2.bstart,
-                                                  cp.L1.bounds, cp.L2.bounds, cp.flags, cp.pos, out, dtested, cat);
+                                                  cp.L1.bounds, cp.L2.bounds, cp.flags, cp.pos, out, cat);
     CF_CHECK(hipGetLastError());
 }
 
+// The call's cell pairs. One synchronisation: for the list's length, the pairs
+// tested and the sets' counts of particles outside the grid (oob1, oob2 or nullptr).
 static int cellpairs_device(const DevLattice& L1, const DevLattice& L2, const int refine[3], const int per[3],
                             const double wrap[3], double max3, double max2, double max1, int min_sep_opt,
-                            int autocorr, CellPairRec** out, int* ncp_out, double* tested, int cat = 0)
+                            int autocorr, const unsigned long long* oob1, const unsigned long long* oob2,
+                            CellPairRec** out, int* ncp_out, double* tested, int cat = 0)
 {
     Engine& E = eng();
     CpPlan cp;
-    if (cellpairs_flag(L1, L2, refine, per, wrap, max3, max2, max1, min_sep_opt, autocorr, cp) != EXIT_SUCCESS)
+    double* dtested = (double*)E.arena.get("cp_tested", sizeof(double) * kTestedSlots);
+    fill_u64(dtested, kTestedSlots);
+    if (cellpairs_flag(L1, L2, refine, per, wrap, max3, max2, max1, min_sep_opt, autocorr, dtested, cp) != EXIT_SUCCESS)
         return EXIT_FAILURE;
     int ncp = 0;
+    double ht[kTestedSlots];
+    unsigned long long h1 = 0, h2 = 0;
     CF_CHECK(hipMemcpyAsync(&ncp, cp.pos + cp.total, sizeof(int), hipMemcpyDeviceToHost, E.stream));
+    CF_CHECK(hipMemcpyAsync(ht, dtested, sizeof ht, hipMemcpyDeviceToHost, E.stream));
+    CF_CHECK(hipMemcpyAsync(&h1, oob1, sizeof h1, hipMemcpyDeviceToHost, E.stream));
+    if (oob2) CF_CHECK(hipMemcpyAsync(&h2, oob2, sizeof h2, hipMemcpyDeviceToHost, E.stream));
     CF_CHECK(hipStreamSynchronize(E.stream));
+    if (check_oob(h1) != EXIT_SUCCESS || check_oob(h2) != EXIT_SUCCESS) return EXIT_FAILURE;
+    *tested = 0;
+    for (int k = 0; k < kTestedSlots; k++) *tested += ht[k];
     CellPairRec* cps = (CellPairRec*)E.arena.get("cp_list", sizeof(CellPairRec) * (ncp + 1));
-    double* dtested = (double*)E.arena.get("cp_tested", sizeof(double));
-    fill_u64(dtested, 1);
-    cellpairs_emit(cp, cps, dtested, cat);
-    CF_CHECK(hipMemcpyAsync(tested, dtested, sizeof(double), hipMemcpyDeviceToHost, E.stream));
-    CF_CHECK(hipStreamSynchronize(E.stream));
+    cellpairs_emit(cp, cps, cat);
     *out = cps;
     *ncp_out = ncp;
     return EXIT_SUCCESS;
@@ -1599,13 +1606,13 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
 
     // ---- gridding on the GPU
     DevLattice L1, L2;
-    if (gridlink_device("l1", g, c.N1, X1, Y1, Z1, W1, esize, L1) != EXIT_SUCCESS) return EXIT_FAILURE;
+    unsigned long long *oob1 = nullptr, *oob2 = nullptr;
+    if (gridlink_device("l1", g, c.N1, X1, Y1, Z1, W1, esize, L1, &oob1) != EXIT_SUCCESS) return EXIT_FAILURE;
     if (!c.autocorr) {
-        if (gridlink_device("l2", g, c.N2, X2, Y2, Z2, W2, esize, L2) != EXIT_SUCCESS) return EXIT_FAILURE;
+        if (gridlink_device("l2", g, c.N2, X2, Y2, Z2, W2, esize, L2, &oob2) != EXIT_SUCCESS) return EXIT_FAILURE;
     } else {
         L2 = L1;
     }
-    const double t_grid = now_s();
     check_interrupt();
 
     // ---- cell pairs
@@ -1617,9 +1624,10 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     CellPairRec* cps = nullptr;
     int ncp = 0;
     double tested = 0;
-    if (cellpairs_device(L1, L2, refine, per, wrap, max3, max2, max1, o->enable_min_sep_opt, c.autocorr, &cps, &ncp,
-                         &tested) != EXIT_SUCCESS)
+    if (cellpairs_device(L1, L2, refine, per, wrap, max3, max2, max1, o->enable_min_sep_opt, c.autocorr, oob1, oob2,
+                         &cps, &ncp, &tested) != EXIT_SUCCESS)
         return EXIT_FAILURE;
+    const double t_grid = now_s();
     check_interrupt();
 
     // ---- launch parameters
@@ -1646,17 +1654,17 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
         set_quant_filter(L2, P);
     }
 
-    // ---- histograms
-    unsigned long long* g_np = (unsigned long long*)E.arena.get("h_np", sizeof(uint64_t) * nslots);
-    double* g_avg = (double*)E.arena.get("h_avg", sizeof(double) * nslots);
-    double* g_w = (double*)E.arena.get("h_w", sizeof(double) * nslots);
-    double* d_edges = (double*)E.arena.get("edges", sizeof(double) * nbin);
-    k_fill_u64<<<(unsigned)((nslots + 255) / 256), 256, 0, E.stream>>>(nslots, g_np, 0ull);
-    k_fill_u64<<<(unsigned)((nslots + 255) / 256), 256, 0, E.stream>>>(nslots, (unsigned long long*)g_avg, 0ull);
-    k_fill_u64<<<(unsigned)((nslots + 255) / 256), 256, 0, E.stream>>>(nslots, (unsigned long long*)g_w, 0ull);
-    CF_CHECK(hipMemcpyAsync(d_edges, rupp_sqr.data(), sizeof(double) * nbin, hipMemcpyHostToDevice, E.stream));
-    unsigned short* d_lut = (unsigned short*)E.arena.get("lut", sizeof(unsigned short) * lut.size());
-    CF_CHECK(hipMemcpyAsync(d_lut, lut.data(), sizeof(unsigned short) * lut.size(), hipMemcpyHostToDevice, E.stream));
+    // ---- histograms (one block: counts, sums of separations, sums of weights),
+    // edges and lookup (one block, one copy)
+    unsigned long long* g_np = (unsigned long long*)E.arena.get("h_all", 3 * sizeof(uint64_t) * nslots);
+    double *g_avg = (double*)(g_np + nslots), *g_w = g_avg + nslots;
+    fill_u64(g_np, 3 * nslots);
+    std::vector<unsigned char> el(sizeof(double) * nbin + sizeof(unsigned short) * lut.size());
+    memcpy(el.data(), rupp_sqr.data(), sizeof(double) * nbin);
+    memcpy(el.data() + sizeof(double) * nbin, lut.data(), sizeof(unsigned short) * lut.size());
+    double* d_edges = (double*)E.arena.get("edges_lut", el.size());
+    unsigned short* d_lut = (unsigned short*)(d_edges + nbin);
+    CF_CHECK(hipMemcpyAsync(d_edges, el.data(), el.size(), hipMemcpyHostToDevice, E.stream));
 
     int nitems = 0;
     TunedRun T;
@@ -1689,22 +1697,15 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
         }
         CF_CHECK(hipEventRecord(E.ev1, E.stream));
     }
-    R.np.assign(nslots, 0);
-    R.avg.assign(nslots, 0.0);
-    R.wavg.assign(nslots, 0.0);
-    CF_CHECK(hipMemcpyAsync(R.np.data(), g_np, sizeof(uint64_t) * nslots, hipMemcpyDeviceToHost, E.stream));
-    CF_CHECK(hipMemcpyAsync(R.avg.data(), g_avg, sizeof(double) * nslots, hipMemcpyDeviceToHost, E.stream));
-    CF_CHECK(hipMemcpyAsync(R.wavg.data(), g_w, sizeof(double) * nslots, hipMemcpyDeviceToHost, E.stream));
+    std::vector<uint64_t> hist(3 * (size_t)nslots);
+    CF_CHECK(hipMemcpyAsync(hist.data(), g_np, 3 * sizeof(uint64_t) * nslots, hipMemcpyDeviceToHost, E.stream));
+    double wsums[2] = {0, 0};
     if (need_w) {
         double* ws = (double*)E.arena.get("wsums", sizeof(double) * 2);
         fill_u64(ws, 2);
         if (c.N1 > 0) k_weight_sums<<<weight_blocks(c.N1), 256, 0, E.stream>>>(c.N1, L1.d4, ws);
         CF_CHECK(hipGetLastError());
-        double h[2];
-        CF_CHECK(hipMemcpyAsync(h, ws, sizeof h, hipMemcpyDeviceToHost, E.stream));
-        CF_CHECK(hipStreamSynchronize(E.stream));
-        R.wsum = h[0];
-        R.wsq = h[1];
+        CF_CHECK(hipMemcpyAsync(wsums, ws, sizeof wsums, hipMemcpyDeviceToHost, E.stream));
     }
     if (c.cell_timer && tuned) {
         // per-cell-pair timings in the order of the cell-pair list (wp_impl:433-463)
@@ -1717,6 +1718,13 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     }
     CF_CHECK(hipStreamSynchronize(E.stream));
     check_interrupt();
+    R.wsum = wsums[0];
+    R.wsq = wsums[1];
+    R.np.assign(hist.begin(), hist.begin() + nslots);
+    R.avg.resize(nslots);
+    R.wavg.resize(nslots);
+    memcpy(R.avg.data(), hist.data() + nslots, sizeof(double) * nslots);
+    memcpy(R.wavg.data(), hist.data() + 2 * nslots, sizeof(double) * nslots);
     float kms = 0, lms = 0;
     CF_CHECK(hipEventElapsedTime(&kms, E.ev0, E.ev1));
     CF_CHECK(hipEventElapsedTime(&lms, E.ev_list, E.ev0));
@@ -1820,22 +1828,21 @@ static int batch_grid(int ncat, std::vector<BatchSet>& sets, size_t esize, std::
                                                                    gbox, big);
     }
     CF_CHECK(hipGetLastError());
-    kb_cellpair_flag<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags);
+    kb_cellpair_flag<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags, d_tested);
     CF_CHECK(hipGetLastError());
     device_scan(flags, pos, T, "ba_pscan");
     int ncp = 0;
     unsigned long long h_oob = 0;
+    std::vector<double> tk(ncat);
+    CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
     CF_CHECK(hipMemcpyAsync(&ncp, pos + T, sizeof(int), hipMemcpyDeviceToHost, E.stream));
     CF_CHECK(hipMemcpyAsync(&h_oob, oob, sizeof h_oob, hipMemcpyDeviceToHost, E.stream));
     CF_CHECK(hipStreamSynchronize(E.stream));
     if (check_oob(h_oob) != EXIT_SUCCESS) return EXIT_FAILURE;
     check_interrupt();
     CellPairRec* cps = (CellPairRec*)E.arena.get("bcp_all", sizeof(CellPairRec) * ((size_t)ncp + 1));
-    kb_cellpair_emit<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags, pos, cps, d_tested);
+    kb_cellpair_emit<<<end.tb0, 256, 0, E.stream>>>(d_sets, ncat, bstart, bounds, flags, pos, cps);
     CF_CHECK(hipGetLastError());
-    std::vector<double> tk(ncat);
-    CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
-    CF_CHECK(hipStreamSynchronize(E.stream));
     *tested = 0;
     for (int k = 0; k < ncat; k++) {
         const BatchSet& s = sets[k];
@@ -2024,12 +2031,14 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
                 return EXIT_FAILURE;
         // cell-pair counts per catalog
         std::vector<int> ncps(ncat);
+        double* d_tested = (double*)E.arena.get("b_tested", sizeof(double) * kTestedSlots);
+        fill_u64(d_tested, kTestedSlots);
         {
             int* d_ncp = (int*)E.arena.get("b_ncp", sizeof(int) * ncat);
             for (int k = 0; k < ncat; k++) {
                 CpPlan cp;
                 if (cellpairs_flag(hl[k], hl[k], refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
-                                   options->enable_min_sep_opt, 1, cp) != EXIT_SUCCESS)
+                                   options->enable_min_sep_opt, 1, d_tested, cp) != EXIT_SUCCESS)
                     return EXIT_FAILURE;
                 k_copy_int<<<1, 64, 0, E.stream>>>(cp.pos + cp.total, d_ncp + k);
             }
@@ -2052,21 +2061,19 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         check_interrupt();
         // concatenated work list, emitted in place
         cps = (CellPairRec*)E.arena.get("bcp_all", sizeof(CellPairRec) * ((size_t)ncp_all + 1));
-        double* d_tested = (double*)E.arena.get("b_tested", sizeof(double) * ncat);
-        fill_u64(d_tested, ncat);
+        {
+            double ht[kTestedSlots];
+            CF_CHECK(hipMemcpyAsync(ht, d_tested, sizeof ht, hipMemcpyDeviceToHost, E.stream));
+            CF_CHECK(hipStreamSynchronize(E.stream));
+            for (double v : ht) tested_all += v;
+        }
         for (int k = 0; k < ncat; k++) {
             if (ncps[k] == 0) continue;
             CpPlan cp;
             if (cellpairs_flag(hl[k], hl[k], refines[k].data(), pers[k].data(), wrap0, rmax, -1, -1,
-                               options->enable_min_sep_opt, 1, cp) != EXIT_SUCCESS)
+                               options->enable_min_sep_opt, 1, d_tested, cp) != EXIT_SUCCESS)
                 return EXIT_FAILURE;
-            cellpairs_emit(cp, cps + cp_off[k], d_tested + k, k);
-        }
-        {
-            std::vector<double> tk(ncat);
-            CF_CHECK(hipMemcpyAsync(tk.data(), d_tested, sizeof(double) * ncat, hipMemcpyDeviceToHost, E.stream));
-            CF_CHECK(hipStreamSynchronize(E.stream));
-            for (int k = 0; k < ncat; k++) tested_all += tk[k];
+            cellpairs_emit(cp, cps + cp_off[k], k);
         }
     }
     const double t_grid = now_s();

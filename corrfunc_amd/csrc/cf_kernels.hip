@@ -587,45 +587,64 @@ __device__ int neighbour_added(const NgbArgs& a, int64_t icell, int k, const int
     return 1;
 }
 
-__global__ void k_cellpair_flag(NgbArgs a, int64_t ncells, int nngb, const int* __restrict__ bs1,
-                                const int* __restrict__ bs2, const double* __restrict__ bd1,
-                                const double* __restrict__ bd2, int* __restrict__ flags)
+// The tests of a kept cell pair.
+__device__ __forceinline__ double pair_tests(const CellPairRec& r, const int* __restrict__ bs1,
+                                             const int* __restrict__ bs2)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= ncells * nngb) return;
-    CellPairRec r = {};
-    flags[t] = neighbour_added(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r);
+    const double n1 = (double)cell_count(bs1, r.c1), n2 = (double)cell_count(bs2, r.c2);
+    return r.same ? n1 * (n1 - 1) * 0.5 : n1 * n2;
 }
 
-// Grid-stride over the candidates; the pairs tested are summed per workgroup
-// (integers below 2^53, exact in any order) and added with one atomic per
-// workgroup, as every atomic on the single counter is serialized.
-__global__ void k_cellpair_emit(NgbArgs a, int64_t ncells, int nngb, const int* __restrict__ bs1,
-                                const int* __restrict__ bs2, const double* __restrict__ bd1,
-                                const double* __restrict__ bd2, const int* __restrict__ flags,
-                                const int* __restrict__ pos, CellPairRec* __restrict__ out,
-                                double* __restrict__ tested, int cat)
+// Adds a workgroup's (256 threads) sum of `my` to *out, one atomic per workgroup
+// (integers below 2^53: exact in any order).
+__device__ __forceinline__ void add_tests(double my, double* __restrict__ out)
 {
     __shared__ double part[4];
-    const int64_t total = ncells * nngb;
-    double my = 0;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        CellPairRec r = {};
-        // (a kept candidate only needs its record again, not the duplicate check)
-        if (flags[t] && eval_neighbour(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r)) {
-            r.pad = cat;
-            out[pos[t]] = r;
-            const double n1 = (double)cell_count(bs1, r.c1), n2 = (double)cell_count(bs2, r.c2);
-            my += r.same ? n1 * (n1 - 1) * 0.5 : n1 * n2;
-        }
-    }
     for (int o = 32; o > 0; o >>= 1) my += __shfl_xor(my, o, 64);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = my;
     __syncthreads();
     if (threadIdx.x == 0) {
         const double s = part[0] + part[1] + part[2] + part[3];
-        if (s != 0) atomicAdd(tested, s);
+        if (s != 0) atomicAdd(out, s);
+    }
+}
+
+// Flags the candidates that are kept; the pairs tested are added to
+// tested[0 .. kTestedSlots - 1], spread because atomics on one address are
+// serialized (~14 ns each).
+constexpr int kTestedSlots = 64;
+__global__ __launch_bounds__(256) void k_cellpair_flag(NgbArgs a, int64_t ncells, int nngb,
+                                                       const int* __restrict__ bs1, const int* __restrict__ bs2,
+                                                       const double* __restrict__ bd1,
+                                                       const double* __restrict__ bd2, int* __restrict__ flags,
+                                                       double* __restrict__ tested)
+{
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    double my = 0;
+    if (t < ncells * nngb) {
+        CellPairRec r = {};
+        const int f = neighbour_added(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r);
+        flags[t] = f;
+        if (f) my = pair_tests(r, bs1, bs2);
+    }
+    add_tests(my, &tested[blockIdx.x % kTestedSlots]);
+}
+
+// The records of the flagged candidates at their scan positions (a kept candidate
+// only needs its record again, not the duplicate check).
+__global__ __launch_bounds__(256) void k_cellpair_emit(NgbArgs a, int64_t ncells, int nngb,
+                                                       const int* __restrict__ bs1, const int* __restrict__ bs2,
+                                                       const double* __restrict__ bd1,
+                                                       const double* __restrict__ bd2, const int* __restrict__ flags,
+                                                       const int* __restrict__ pos, CellPairRec* __restrict__ out,
+                                                       int cat)
+{
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t >= ncells * nngb || !flags[t]) return;
+    CellPairRec r = {};
+    if (eval_neighbour(a, t / nngb, (int)(t % nngb), bs1, bs2, bd1, bd2, &r)) {
+        r.pad = cat;
+        out[pos[t]] = r;
     }
 }
 
