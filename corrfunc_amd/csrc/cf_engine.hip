@@ -1066,13 +1066,18 @@ static int tuned_shape(int batch, PairParams& P, int nslots, int nbin, TunedShap
     }
     // Launch shape for a workgroup of `thr` threads: LDS histogram replication
     // R (power of 2, <= 32, histograms <= the LDS limit less 24 KiB) = the
-    // largest that keeps min(16, best achievable) waves per CU resident (on-sky
-    // modes: the best achievable, since their survivors' FP64 decision needs
-    // the latency hiding more than the histogram needs copies; measured on
-    // DDrppi_mocks, R 4 at 16 waves is 15 % slower than R 2 at 24, while
-    // DDrppi gains 4 %); the primaries cache where it costs no resident
-    // workgroup; `per_cu` = resident workgroups per CU (registers and LDS),
-    // which is also how many persistent workgroups per CU are launched.
+    // largest that keeps min(16, best achievable) waves per CU resident; more than
+    // kCostlyCopies copies only where they cost neither a wave nor the primaries
+    // cache: up to 8 copies are worth waves (DDrppi on clumps 22.5 / 15.7 / 12.2 ms
+    // with 2 / 4 / 8), more are not (batched DD 182 ms with 16 copies at 16 waves, 170
+    // with 8 at 24; DDsmu of 300k points 1.56 ms with 16 and no cache, 1.30 with 8 and
+    // the cache). On-sky modes keep the best achievable waves throughout, since
+    // their survivors' FP64 decision needs the latency hiding more than the
+    // histogram needs copies (DDrppi_mocks 27.1 ms with 4 at 16 waves, 25.4 with 2 at
+    // 24). The primaries cache where it costs no resident workgroup; `per_cu` =
+    // resident workgroups per CU (registers and LDS), which is also how many
+    // persistent workgroups per CU are launched.
+    constexpr int kCostlyCopies = 8;
     struct Shape {
         int threads, nwaves, R, prim, per_cu;
         size_t lds;
@@ -1101,6 +1106,7 @@ static int tuned_shape(int batch, PairParams& P, int nslots, int nbin, TunedShap
             if ((size_t)regions * nslots * per_slot * r > E.lds_max - 24 * 1024) break;
             if (lds_for(r) > E.lds_max) break;  // (the workgroup's queues included)
             if (resident(lds_for(r)) * sh.nwaves < target) break;
+            if (r > kCostlyCopies && resident(lds_for(r) + lds_prim) * sh.nwaves < best) break;
             R = r;
         }
         if (const char* rc = getenv("CORRFUNC_AMD_HIST_COPIES")) {
