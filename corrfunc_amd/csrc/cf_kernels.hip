@@ -1511,6 +1511,15 @@ __device__ __forceinline__ void reg_groups(const PairParams& P, const CellPairRe
     }
 }
 
+// One lane's value from its neighbour in the row of 16 lanes (a DPP row rotation).
+static_assert(kGroup == 16, "a group of secondaries is held by a row of 16 lanes");
+__device__ __forceinline__ double row_next(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x121, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x121, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
 // One work item of the tuned kernel (see the comment above kQueues).
 template <int MODE, int R2F, bool GH, int DP, int FL>
 __device__ __forceinline__ void process_item(const PairParams& P, const DevLattice* l1p, const DevLattice* l2p,
@@ -1686,6 +1695,37 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
                     reg_groups<MODE, R2F, 3>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
                 else if (nb == 4)
                     reg_groups<MODE, R2F, 4>(P, cpp, l1p, i, ivalid, xpos, ypos, zpos, ds, m, jb0, e2, k0, touch, S);
+            }
+        }
+        // DDsmu's dense path: every row of 16 lanes holds a group's secondaries and
+        // rotates them, so the lanes of a histogram update have 16 different
+        // secondaries. With one secondary for all lanes, compact chunks put many lanes
+        // into one (s, mu) slot, and the same-address atomics serialize: 31 % of the
+        // cycles on clustered data x randoms, 389 -> 314 ms; the rotation's 8 moves
+        // cost 4 % where the points are uniform. (DDrppi, whose pi columns already
+        // spread a compact chunk: 3 % slower; on-sky modes are bound by the decision's
+        // arithmetic.)
+        constexpr bool rotate = MODE == MODE_SMU;
+        if constexpr (rotate) {
+            const int r = lane & (kGroup - 1);
+            while (mdense) {
+                const int g = __builtin_ctzll(mdense);
+                mdense &= mdense - 1;
+                const int j0 = s2 + (g0 + g) * kGroup;
+                int j = j0 + r;
+                double4 cur = d4_2[min(j, e2 - 1)];
+                int left = kGroup;
+                for (;;) {
+                    exact_pair<MODE, R2F, GH, FL>(P, cpp, l1p, i, j > ilim && j < e2, xpos, ypos, zpos, wi, cur.x,
+                                                  cur.y, cur.z, fl_w<FL>(P) ? cur.w : 0.0, S);
+                    if (--left == 0) break;
+                    cur.x = row_next(cur.x);
+                    cur.y = row_next(cur.y);
+                    cur.z = row_next(cur.z);
+                    if (fl_w<FL>(P)) cur.w = row_next(cur.w);
+                    // (row_ror 1: lane l takes lane l - 1's)
+                    j = j0 + ((j - j0 + kGroup - 1) & (kGroup - 1));
+                }
             }
         }
         while (mdense) {
