@@ -148,6 +148,7 @@ struct Engine {
     // autotuner
     bool autotune = false;
     bool tuning = false;            // inside a candidate run
+    bool full_list = false;         // the work list takes every cell pair (a batch graph sizes its list by it)
     int force_R = 0;                // histogram replication override (0: automatic)
     int force_fetch = 0;            // queue batch override (0: CORRFUNC_AMD_FETCH or the work-list rule)
     int last_autotuned = 0;         // 0 off, 1 cached choice, 2 tuned by this call
@@ -1200,7 +1201,7 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
     const int per_cu = ts.per_cu;
     const long max_blocks = (long)E.ncu * per_cu;
     // (per-cell-pair timings need every cell pair in the list)
-    const int light = !gh && !timed && P.dense_mode == 0 && tested <= kLightMean * ncp &&
+    const int light = !gh && !timed && !E.full_list && P.dense_mode == 0 && tested <= kLightMean * ncp &&
                               launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, true)
                           ? kLightPairs
                           : 0;
@@ -2282,9 +2283,12 @@ static int bg_create(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
     {
         struct config_options oc = *options;
         std::vector<CallOut> outs;
-        const int sched = E.sched_kind;
+        // (the graph has no light kernel: its list takes every cell pair)
+        struct FullList {
+            FullList() { eng().full_list = true; }
+            ~FullList() { eng().full_list = false; }
+        } full;
         if (run_batch(ncat, ND, X, Y, Z, W, binfile, &oc, extra, outs) != EXIT_SUCCESS) return EXIT_FAILURE;
-        (void)sched;
     }
     const double ncp0 = (double)E.last.num_cell_pairs, items0 = (double)E.last.num_work_items;
     const int fetch0 = E.last.queue_fetch;

@@ -65,3 +65,21 @@ def test_batch_of_unequal_catalogs(engine, oracle, dtype):
         assert np.array_equal(got["npairs"][1:], want["npairs"][1:])
         for k in ("ravg", "weightavg"):
             assert np.allclose(got[k][1:], want[k][1:], rtol=1e-10, atol=0)
+
+
+def test_graph_of_sparse_catalogs(engine, oracle):
+    """A captured batch has no light kernel: its work list takes every cell pair."""
+    os.environ["CORRFUNC_AMD_DENSE"] = "0"
+    _lib.set_engine(_lib.ENGINE_TUNED)
+    cats = [_sparse(9000, c, np.float64, 50 + c) for c in (0, 40, 0)]
+    dev = [[_lib.DeviceArray(a) for a in x] for x in cats]
+    o = dict(periodic=True, boxsize=L, need_avg_sep=True)
+    g = _lib.BatchGraph([tuple(d) for d in dev], BINS, options=_abi.make_options(**o))
+    try:
+        for _ in range(2):
+            for x, got in zip(cats, g.launch()):
+                want = run(oracle, "countpairs", "oracle_", options=_abi.make_options(**o),
+                           **mode_kwargs("countpairs", x, bins=BINS, L=L))
+                assert_same("countpairs", got, want, what="graph")
+    finally:
+        g.close()
