@@ -98,7 +98,8 @@ __global__ __launch_bounds__(256) void kb_build_small(const BatchSet* __restrict
         return;
     }
     build_cell<T, 64, kSmallBins>(c, lane, (const T*)s.X, (const T*)s.Y, (const T*)s.Z, (const T*)s.W, s.g, bs, idx,
-                                  keys, d4, q, bounds + 6 * s.c0, gbox + 6 * s.c0, hist[wave], nullptr);
+                                  keys, d4, q, bounds + 6 * s.c0, gbox + 6 * s.c0, nullptr,
+                                  hist[wave], nullptr);
 }
 template <typename T>
 __global__ __launch_bounds__(kBigThreads) void kb_build_big(const BatchSet* __restrict__ sets, int ncat,
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(kBigThreads) void kb_build_big(const BatchSet* __re
         const BatchSet& s = sets[lo];
         build_cell<T, kBigThreads, kBigBins>(gc - s.c0, threadIdx.x, (const T*)s.X, (const T*)s.Y, (const T*)s.Z,
                                              (const T*)s.W, s.g, bstart + s.c0, idx, keys, d4, q, bounds + 6 * s.c0,
-                                             gbox + 6 * s.c0, hist, red);
+                                             gbox + 6 * s.c0, nullptr, hist, red);
         __syncthreads();
     }
 }

@@ -160,14 +160,16 @@ __global__ __launch_bounds__(256) void k_bg_build_small(const T* X, const T* Y, 
                                                         const BgCat* cat, DevLattice B, const int* idx, int* keys,
                                                         int* big)
 {
-    build_small(cat->ncells, X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, big);
+    build_small(cat->ncells, X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, nullptr,
+                big);
 }
 template <typename T>
 __global__ __launch_bounds__(kBigThreads) void k_bg_build_big(const T* X, const T* Y, const T* Z, const T* W,
                                                               const BgCat* cat, DevLattice B, const int* idx,
                                                               int* keys, const int* big)
 {
-    build_big(X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, big);
+    build_big(X, Y, Z, W, cat->g, B.bstart, idx, keys, B.d4, B.q, B.bounds, B.gbox, nullptr,
+                big);
 }
 
 // Candidates (cell, neighbour) over the captured capacity `cap`; those beyond

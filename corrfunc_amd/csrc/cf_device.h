@@ -62,7 +62,11 @@ struct DevLattice {
     unsigned qrange;           // filter: pass iff (dq^2 + qlo_neg) mod 2^32 < qrange
     int qlo_neg;
     int qz;                    // projected modes: pass iff |dqz| < qz
-    int qpad_;
+    // On-sky (rp, pi): 2 |x|^2 per particle (FP32, kQPad entries of padding) and the
+    // constants of the line-of-sight test of the filter (qpass); nullptr otherwise.
+    int los_pad_;
+    float *rr;
+    float los_c1, los_c0, los_a0, los_t0;
     int *bstart;               // [ncells + 1] cell starts
     double *gbox;              // [(n/kGroup + ncells + 1)*6] the groups' boxes, x lo,hi, y lo,hi, z lo,hi
     double *bounds;            // [ncells*6] x lo,hi, y lo,hi, z lo,hi

@@ -440,7 +440,8 @@ static double grid_qinv(const GridSpec& g) { return (double)kQMax / (fmax(g.xbs,
 // Counting-sort gridding launched on the stream without waiting: particles
 // outside the grid are counted into *oob (zeroed by the caller) and skipped.
 static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n, const void* X, const void* Y,
-                           const void* Z, const void* W, size_t esize, DevLattice& L, unsigned long long* oob)
+                           const void* Z, const void* W, size_t esize, DevLattice& L, unsigned long long* oob,
+                           bool los = false)
 {
     Engine& E = eng();
     L.nx = g.nx; L.ny = g.ny; L.nz = g.nz;
@@ -467,6 +468,7 @@ static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n,
     L.q = (uint2*)E.arena.get(tag + "_q", sizeof(uint2) * (n + kQPad));
     L.bounds = (double*)E.arena.get(tag + "_bounds", sizeof(double) * 6 * L.ncells);
     L.gbox = (double*)E.arena.get(tag + "_gbox", sizeof(double) * 6 * (n / kGroup + L.ncells + 1));
+    L.rr = los ? (float*)E.arena.get(tag + "_rr", sizeof(float) * (n + kQPad)) : nullptr;
     fill_i32(counts, nb + 1, 0);
     fill_i32(big, 1, 0);
     GridArgs ga{g.xmin, g.ymin, g.zmin, g.xinv, g.yinv, g.zinv, g.xbs, g.ybs, g.zbs, g.nx, g.ny, g.nz, L.qinv};
@@ -490,21 +492,21 @@ static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n,
     if (esize == 4)
         k_build_small<float><<<sb, 256, 0, E.stream>>>(L.ncells, (const float*)X, (const float*)Y, (const float*)Z,
                                                         (const float*)W, ga, L.bstart, idx, rank, L.d4, L.q,
-                                                        L.bounds, L.gbox, big);
+                                                        L.bounds, L.gbox, L.rr, big);
     else
         k_build_small<double><<<sb, 256, 0, E.stream>>>(L.ncells, (const double*)X, (const double*)Y,
                                                          (const double*)Z, (const double*)W, ga, L.bstart, idx,
-                                                         rank, L.d4, L.q, L.bounds, L.gbox, big);
+                                                         rank, L.d4, L.q, L.bounds, L.gbox, L.rr, big);
     CF_CHECK(hipGetLastError());
     if (bb > 0) {
         if (esize == 4)
             k_build_big<float><<<bb, kBigThreads, 0, E.stream>>>((const float*)X, (const float*)Y, (const float*)Z,
                                                                   (const float*)W, ga, L.bstart, idx, rank, L.d4,
-                                                                  L.q, L.bounds, L.gbox, big);
+                                                                  L.q, L.bounds, L.gbox, L.rr, big);
         else
             k_build_big<double><<<bb, kBigThreads, 0, E.stream>>>((const double*)X, (const double*)Y,
                                                                    (const double*)Z, (const double*)W, ga, L.bstart,
-                                                                   idx, rank, L.d4, L.q, L.bounds, L.gbox, big);
+                                                                   idx, rank, L.d4, L.q, L.bounds, L.gbox, L.rr, big);
         CF_CHECK(hipGetLastError());
     }
     return EXIT_SUCCESS;
@@ -522,12 +524,13 @@ static int check_oob(unsigned long long n_oob)
 // Gridding of one set of a call; its count of particles outside the grid stays on
 // the device (*oob) until the call's next synchronisation.
 static int gridlink_device(const std::string& tag, const GridSpec& g, int64_t n, const void* X, const void* Y,
-                           const void* Z, const void* W, size_t esize, DevLattice& L, unsigned long long** oob)
+                           const void* Z, const void* W, size_t esize, DevLattice& L, unsigned long long** oob,
+                           bool los)
 {
     Engine& E = eng();
     *oob = (unsigned long long*)E.arena.get(tag + "_oob", 8);
     fill_u64(*oob, 1);
-    return gridlink_launch(tag, g, n, X, Y, Z, W, esize, L, *oob);
+    return gridlink_launch(tag, g, n, X, Y, Z, W, esize, L, *oob, los);
 }
 
 // Workgroups of k_weight_sums: 8 records a thread, at most 512 (two atomics each).
@@ -858,10 +861,12 @@ static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, con
         // NFW halos -0.6 %, DD and DDsmu equal)
         P.dense_stride = ds ? atoi(ds) : 0;
         const char* df = getenv("CORRFUNC_AMD_DENSE_FRAC");
-        // measured (bench.py --sweep CORRFUNC_AMD_DENSE_FRAC): DDsmu cross
-        // (workload 5) 2.71 s at 0.35, 2.60 s at 0.2-0.25, 3.18 s at 0; DDrppi
-        // and DD within 2 % from 0.2 to 0.5
-        P.dense_frac = df ? (float)atof(df) : 0.25f;
+        // per group of secondaries; 0.1 to 0.15 cost DD, xi and batches 5-20 %, 0.4 to
+        // 0.5 gain 1 % on DDrppi and DDsmu and cost xi 5 %. On-sky (rp, pi): the
+        // estimate is of the 3-D limit, of which the filter's line-of-sight test
+        // leaves a third, so only groups nearly inside go past it (25.5 ms at 0.25,
+        // 21.7 at 0.85)
+        P.dense_frac = df ? (float)atof(df) : (mode == MODE_RPPI_MOCKS ? 0.85f : 0.25f);
         const char* qb = getenv("CORRFUNC_AMD_QBLOCK_LOG2");
         // blocks of 32 items per sub-queue (measured, bench.py --sweep
         // CORRFUNC_AMD_QBLOCK_LOG2=0..8): DDsmu cross -1.8 %, DDrppi -1.5 %, DD and xi
@@ -874,13 +879,12 @@ static void build_params(int mode, int isa_id, int nbin, int n2, int nslots, con
 
 }
 
-// Device copy of the (primary, secondary) lattice pair of a single call.
 // Thresholds of the integer pair filter of a secondary set (quantum 1/L.qinv).
 // Rounding both positions of a pair to the nearest quantum moves their
 // difference by at most one quantum per axis, so in quanta a pair at distance d
 // has |dq| <= d*qinv + sqrt(3) (3-D) and |dqz| <= |dz|*qinv + 1; the bounds
 // below add slack to these, so every pair the FP64 test can accept passes.
-static void set_quant_filter(DevLattice& L, const PairParams& P)
+static void set_quant_filter(DevLattice& L, const PairParams& P, double r2max = 0.0)
 {
     const bool is2d = P.mode == MODE_RPPI || P.mode == MODE_WP;
     const double rhi = sqrt(P.sqr_rmax) * (1.0 + 1e-9) * L.qinv + 2.0;
@@ -890,8 +894,20 @@ static void set_quant_filter(DevLattice& L, const PairParams& P)
     L.qrange = (unsigned)(hi - lo);
     L.qlo_neg = -(int)lo;
     L.qz = is2d ? (int)ceil(P.pimax * (1.0 + 1e-9) * L.qinv + 1.0) + 1 : 0;
+    L.los_c1 = L.los_c0 = L.los_a0 = L.los_t0 = 0.0f;
+    // (beyond FP32's range the terms stay 0, which passes every pair)
+    if (L.rr && r2max > 0 && r2max < 1e15) {
+        // qpass's test, both sides times 4; u = (s^2 - slack - rpmax^2) (1 - 1e-4)
+        const double h = 1.0 / L.qinv, smax = sqrt(P.sqr_rmax);
+        const double slack = 4.0 * h * smax + 4.0 * h * h + 1e-5 * P.sqr_rmax;
+        L.los_c1 = (float)(4.0 * (1.0 - 1e-4) * h * h);
+        L.los_c0 = (float)(4.0 * (1.0 - 1e-4) * (lo * h * h - slack - P.sqr_rpmax * (1.0 + 1e-9)));
+        L.los_a0 = (float)((P.sqr_rmax + 0x1p-20 * r2max) * (1.0 + 1e-6));
+        L.los_t0 = (float)(0x1p-19 * r2max);
+    }
 }
 
+// Device copy of the (primary, secondary) lattice pair of a single call.
 static const DevLattice* lats_for(const DevLattice& L1, const DevLattice& L2)
 {
     Engine& E = eng();
@@ -1614,9 +1630,9 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
     // ---- gridding on the GPU
     DevLattice L1, L2;
     unsigned long long *oob1 = nullptr, *oob2 = nullptr;
-    if (gridlink_device("l1", g, c.N1, X1, Y1, Z1, W1, esize, L1, &oob1) != EXIT_SUCCESS) return EXIT_FAILURE;
+    if (gridlink_device("l1", g, c.N1, X1, Y1, Z1, W1, esize, L1, &oob1, mode == MODE_RPPI_MOCKS) != EXIT_SUCCESS) return EXIT_FAILURE;
     if (!c.autocorr) {
-        if (gridlink_device("l2", g, c.N2, X2, Y2, Z2, W2, esize, L2, &oob2) != EXIT_SUCCESS) return EXIT_FAILURE;
+        if (gridlink_device("l2", g, c.N2, X2, Y2, Z2, W2, esize, L2, &oob2, mode == MODE_RPPI_MOCKS) != EXIT_SUCCESS) return EXIT_FAILURE;
     } else {
         L2 = L1;
     }
@@ -1657,8 +1673,10 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
             P.zreach = sqrt(P.sqr_rmax);
             P.near_lo2 = P.sqr_rmax - (1e-9 * P.sqr_rmax + 1e-9 * max_sep * coord_scale);
         }
-        set_quant_filter(L1, P);
-        set_quant_filter(L2, P);
+        double r2max = 0;  // no |x|^2 exceeds it
+        for (int d = 0; d < 3; d++) r2max += fmax(ext[d] * ext[d], ext[3 + d] * ext[3 + d]);
+        set_quant_filter(L1, P, r2max);
+        set_quant_filter(L2, P, r2max);
     }
 
     // ---- histograms (one block: counts, sums of separations, sums of weights),

@@ -285,8 +285,8 @@ __device__ __forceinline__ void build_cell(int64_t c, int tid, const T* __restri
                                            const T* __restrict__ Z, const T* __restrict__ W, const GridArgs& g,
                                            const int* __restrict__ bstart, const int* __restrict__ idx,
                                            int* __restrict__ keys, double4* d4, uint2* __restrict__ q,
-                                           double* __restrict__ bounds, double* __restrict__ gbox, int* hist,
-                                           double* red)
+                                           double* __restrict__ bounds, double* __restrict__ gbox,
+                                           float* __restrict__ rr, int* hist, double* red)
 {
     const int s = bstart[c], n = bstart[c + 1] - s;
     const int lane = tid & 63;
@@ -343,6 +343,7 @@ __device__ __forceinline__ void build_cell(int64_t c, int tid, const T* __restri
             const int pos = s + atomicAdd(&hist[keys[s + k]], 1);
             d4[pos] = make_double4(xv, yv, zv, W ? (double)W[i] : 0.0);
             q[pos] = quantize_pos(xv - ox, yv - oy, zv - oz, g.qinv);
+            if (rr) rr[pos] = (float)(2.0 * (xv * xv + yv * yv + zv * zv));
         }
     }
     // cell bounds (min / max are exact, so the order of the reduction does not
@@ -403,7 +404,7 @@ __device__ __forceinline__ void build_cell(int64_t c, int tid, const T* __restri
 template <typename T>
 __device__ __forceinline__ void build_small(int64_t ncells, const T* X, const T* Y, const T* Z, const T* W,
                                             const GridArgs& g, const int* bstart, const int* idx, int* keys,
-                                            double4* d4, uint2* q, double* bounds, double* gbox, int* big)
+                                            double4* d4, uint2* q, double* bounds, double* gbox, float* rr, int* big)
 {
     __shared__ int hist[4][kSmallBins];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -413,35 +414,38 @@ __device__ __forceinline__ void build_small(int64_t ncells, const T* X, const T*
         if (lane == 0) big[1 + atomicAdd(big, 1)] = (int)c;
         return;
     }
-    build_cell<T, 64, kSmallBins>(c, lane, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, hist[wave], nullptr);
+    build_cell<T, 64, kSmallBins>(c, lane, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, rr,
+                                      hist[wave], nullptr);
 }
 template <typename T>
 __device__ __forceinline__ void build_big(const T* X, const T* Y, const T* Z, const T* W, const GridArgs& g,
                                           const int* bstart, const int* idx, int* keys, double4* d4, uint2* q,
-                                          double* bounds, double* gbox, const int* big)
+                                          double* bounds, double* gbox, float* rr, const int* big)
 {
     __shared__ int hist[kBigBins];
     __shared__ double red[6 * kBigThreads / 64];
     const int nbig = big[0];
     for (int t = blockIdx.x; t < nbig; t += gridDim.x) {
         build_cell<T, kBigThreads, kBigBins>(big[1 + t], threadIdx.x, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds,
-                                             gbox, hist, red);
+                                             gbox, rr, hist, red);
         __syncthreads();
     }
 }
 template <typename T>
 __global__ __launch_bounds__(256) void k_build_small(int64_t ncells, const T* X, const T* Y, const T* Z, const T* W,
                                                      GridArgs g, const int* bstart, const int* idx, int* keys,
-                                                     double4* d4, uint2* q, double* bounds, double* gbox, int* big)
+                                                     double4* d4, uint2* q, double* bounds, double* gbox, float* rr,
+                                                     int* big)
 {
-    build_small(ncells, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, big);
+    build_small(ncells, X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, rr, big);
 }
 template <typename T>
 __global__ __launch_bounds__(kBigThreads) void k_build_big(const T* X, const T* Y, const T* Z, const T* W, GridArgs g,
                                                            const int* bstart, const int* idx, int* keys, double4* d4,
-                                                           uint2* q, double* bounds, double* gbox, const int* big)
+                                                           uint2* q, double* bounds, double* gbox, float* rr,
+                                                           const int* big)
 {
-    build_big(X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, big);
+    build_big(X, Y, Z, W, g, bstart, idx, keys, d4, q, bounds, gbox, rr, big);
 }
 
 // Sums of the weights and of their squares over the grid-ordered records
@@ -1306,7 +1310,17 @@ __device__ __forceinline__ void drain_queue2(const PairParams& P, const CellPair
 // the same on (dqx, dqy) and |dqz| < zq, as (dqz + zq - 1) unsigned < 2 zq - 1
 // with zoff = zq - 1 - qz. Differences fit 16 bits and sums of squares 32 bits
 // (|q| <= kQMax), so the only rounding is that of the positions themselves.
+//
+// On-sky (rp, pi) adds a test of rp: with l = x_i + x_j, s.l = |x_j|^2 - |x_i|^2 and
+// |l|^2 = 2 |x_i|^2 + 2 |x_j|^2 - s^2, so rp^2 < rpmax^2 means (s^2 - rpmax^2) |l|^2 <
+// (s.l)^2. In FP32 from the quantized s^2 and the stored 2 |x|^2: the left side is
+// taken too small (s^2 less the quantization's 4 h smax, |l|^2 with smax^2 for s^2 and
+// less 2^-20 of the largest |x|^2, at least 0) and |s.l| too large (by 2^-20 of it),
+// which covers the rounding, so every pair the FP64 test can accept passes (NaN passes). Of the
+// pairs within the 3-D limit 64 % are out of rp range (rpmax 25, pimax 40), and
+// eight instructions here replace their share of a decision of about 85.
 struct QFilter {
+    float los_r, los_a, los_c1, los_c0, los_t0;  // 2 |x_i|^2 and the test's terms
     unsigned qxy;
     int qz, qlo, zoff;
     unsigned qrange, zspan;
@@ -1314,7 +1328,7 @@ struct QFilter {
 };
 // The wave's mask of lanes whose pair with secondary s (index j) survives.
 template <int MODE, bool SAME>
-__device__ __forceinline__ unsigned long long qpass(const QFilter& f, uint2 s, int j)
+__device__ __forceinline__ unsigned long long qpass(const QFilter& f, uint2 s, float rj, int j)
 {
     const short2v d = __builtin_bit_cast(short2v, s.x) - __builtin_bit_cast(short2v, f.qxy);
     unsigned long long m;
@@ -1326,6 +1340,11 @@ __device__ __forceinline__ unsigned long long qpass(const QFilter& f, uint2 s, i
         const int dz = (int)s.y - f.qz;
         const int r = __builtin_amdgcn_sdot2(d, d, __mul24(dz, dz) + f.qlo, false);
         m = __builtin_amdgcn_ballot_w64((unsigned)r < f.qrange);
+        if (MODE == MODE_RPPI_MOCKS) {
+            const float u = fmaf((float)(unsigned)r, f.los_c1, f.los_c0);
+            const float t = fabsf(rj - f.los_r) + f.los_t0;
+            m &= __builtin_amdgcn_ballot_w64(!(u * fmaxf(rj + f.los_a, 0.0f) > t * t));
+        }
     }
     // same cell: the lane's own j > i (lanes without a primary have quantized
     // positions no secondary passes)
@@ -1358,13 +1377,19 @@ __device__ __forceinline__ void enqueue(unsigned* qe, unsigned long long m, unsi
 // A block of kBlockJ quantized secondaries in scalar registers.
 struct QBlock {
     uint2 s[kBlockJ];
+    float r[kBlockJ];  // on-sky (rp, pi)
 };
-__device__ __forceinline__ QBlock qload(KUint* qs, int jb)
+typedef const __attribute__((address_space(4))) float KFloat;
+template <int MODE>
+__device__ __forceinline__ QBlock qload(KUint* qs, KFloat* rs, int jb)
 {
     KUint* p = qs + 2 * (int64_t)jb;
     QBlock b;
 #pragma unroll
-    for (int t = 0; t < kBlockJ; t++) b.s[t] = make_uint2(p[2 * t], p[2 * t + 1]);
+    for (int t = 0; t < kBlockJ; t++) {
+        b.s[t] = make_uint2(p[2 * t], p[2 * t + 1]);
+        b.r[t] = MODE == MODE_RPPI_MOCKS ? rs[(int64_t)jb + t] : 0.0f;
+    }
     return b;
 }
 
@@ -1377,7 +1402,7 @@ __device__ __forceinline__ void qblock(const QFilter& f, const QBlock& b, int jb
     unsigned long long m[kBlockJ];
 #pragma unroll
     for (int t = 0; t < kBlockJ; t++) {
-        m[t] = qpass<MODE, SAME>(f, b.s[t], jb + t);
+        m[t] = qpass<MODE, SAME>(f, b.s[t], b.r[t], jb + t);
         if (PARTIAL) m[t] = t < nlive ? m[t] : 0ull;
     }
     const unsigned e0 = ((unsigned)(jb - jbase) << 6) | (unsigned)lane_id();
@@ -1392,20 +1417,20 @@ __device__ __forceinline__ void qblock(const QFilter& f, const QBlock& b, int jb
 // two register blocks so that each block is loaded one block ahead (q is padded
 // by kQPad entries, so the look-ahead stays inside the array).
 template <int MODE, bool SAME, int DRAIN>
-__device__ __forceinline__ int qscan(const QFilter& f, KUint* qs, int jb, int jhi, QBlock& a, unsigned* qe,
+__device__ __forceinline__ int qscan(const QFilter& f, KUint* qs, KFloat* rs, int jb, int jhi, QBlock& a, unsigned* qe,
                                      unsigned head, unsigned& tail, int jbase)
 {
     int nfull = (jhi - jb) / kBlockJ;
     for (;;) {
         if (nfull <= 0 || tail - head >= DRAIN) return jb;
-        const QBlock b = qload(qs, jb + kBlockJ);
+        const QBlock b = qload<MODE>(qs, rs, jb + kBlockJ);
         qblock<MODE, SAME, false>(f, a, jb, kBlockJ, qe, tail, jbase);
         jb += kBlockJ;
         if (--nfull <= 0 || tail - head >= DRAIN) {
             a = b;
             return jb;
         }
-        a = qload(qs, jb + kBlockJ);
+        a = qload<MODE>(qs, rs, jb + kBlockJ);
         qblock<MODE, SAME, false>(f, b, jb, kBlockJ, qe, tail, jbase);
         jb += kBlockJ;
         --nfull;
@@ -1600,6 +1625,15 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
     }
     KDouble* ds = (KDouble*)(const void*)d4_2;
     KUint* qs = (KUint*)(const void*)L2.q;
+    KFloat* rs = nullptr;
+    if (MODE == MODE_RPPI_MOCKS) {
+        rs = (KFloat*)(const void*)L2.rr;
+        f.los_r = (float)(2.0 * (xpos * xpos + ypos * ypos + zpos * zpos));
+        f.los_a = f.los_r - L2.los_a0;
+        f.los_c1 = L2.los_c1;
+        f.los_c0 = L2.los_c0;
+        f.los_t0 = L2.los_t0;
+    }
     constexpr int kDrain = 64 * DP;
     for (int g0 = glo; g0 < ghi; g0 += 64) {
         // lane l tests group g0 + l against the chunk's box: out of reach,
@@ -1646,7 +1680,27 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
             const double near2 = is2d ? nx * nx + ny * ny : nx * nx + ny * ny + nz * nz;
             const double far2 = is2d ? fx * fx + fy * fy : fx * fx + fy * fy + fz * fz;
             // the margins cover the rounding of the pairs' own separations
-            const bool live = have && near2 <= P.sqr_rmax * (1.0 + 1e-9) && nz <= P.zreach * (1.0 + 1e-9) + P.box_margin;
+            bool live = have && near2 <= P.sqr_rmax * (1.0 + 1e-9) && nz <= P.zreach * (1.0 + 1e-9) + P.box_margin;
+            if (MODE == MODE_RPPI_MOCKS) {
+                // the filter's line-of-sight test (QFilter) on the boxes' ranges of |x|^2, and
+                // pi < pimax by (s.l)^2 < pimax^2 |l|^2
+                const double x0s = x0 * x0, x1s = x1 * x1, y0s = y0 * y0, y1s = y1 * y1, z0s = z0 * z0, z1s = z1 * z1;
+                const double hi2 = fmax(x0s, x1s) + fmax(y0s, y1s) + fmax(z0s, z1s);
+                const double lo2 = (x0 * x1 > 0 ? fmin(x0s, x1s) : 0.0) + (y0 * y1 > 0 ? fmin(y0s, y1s) : 0.0) +
+                                   (z0 * z1 > 0 ? fmin(z0s, z1s) : 0.0);
+                double hi1 = 0, lo1 = 0;
+#pragma unroll
+                for (int d = 0; d < 6; d += 2) {
+                    const double u = A[d] * A[d], v = A[d + 1] * A[d + 1];
+                    hi1 += fmax(u, v);
+                    lo1 += A[d] * A[d + 1] > 0 ? fmin(u, v) : 0.0;
+                }
+                const double slack = 1e-9 * (hi1 + hi2);
+                const double tmax = fmax(hi2 - lo1, hi1 - lo2) + slack, tmin = fmax(fmax(lo2 - hi1, lo1 - hi2) - slack, 0.0);
+                const double lmin = fmax(2.0 * (lo1 + lo2) - P.sqr_rmax - slack, 0.0), lmax = 2.0 * (hi1 + hi2) + slack;
+                live = live && !((near2 * (1.0 - 1e-9) - P.sqr_rpmax) * lmin > tmax * tmax) &&
+                       !(tmin * tmin > P.sqr_mu_max * lmax);
+            }
             double num = P.sqr_rmax - near2, den = far2 - near2;
             bool dns = num >= (double)P.dense_frac * den;
             if (is2d) {
@@ -1753,16 +1807,16 @@ __device__ __forceinline__ void process_item(const PairParams& P, const DevLatti
             if (jb >= jhi) {
                 if (msparse) {
                     next_run(msparse, jbase, e2, jb, jhi);
-                    a = qload(qs, jb);
+                    a = qload<MODE>(qs, rs, jb);
                 } else {
                     last = true;
                 }
             }
             if (!last) {
                 if (same)
-                    jb = qscan<MODE, true, kDrain>(f, qs, jb, jhi, a, qe, head, tail, jbase);
+                    jb = qscan<MODE, true, kDrain>(f, qs, rs, jb, jhi, a, qe, head, tail, jbase);
                 else
-                    jb = qscan<MODE, false, kDrain>(f, qs, jb, jhi, a, qe, head, tail, jbase);
+                    jb = qscan<MODE, false, kDrain>(f, qs, rs, jb, jhi, a, qe, head, tail, jbase);
                 if (jb < jhi && jb + kBlockJ > jhi && tail - head < kDrain) {
                     // the last, partial block
                     if (same)
