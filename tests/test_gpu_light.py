@@ -83,3 +83,18 @@ def test_graph_of_sparse_catalogs(engine, oracle):
                 assert_same("countpairs", got, want, what="graph")
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("rmax", [1.45, 2.6, 30.0])
+def test_scans_of_every_depth(engine, oracle, rmax):
+    """27 million candidate cell pairs (a scan of scanned block sums), 4 million, and a few hundred
+    (one block)."""
+    os.environ["CORRFUNC_AMD_DENSE"] = "0"
+    _lib.set_engine(_lib.ENGINE_TUNED)
+    X = _sparse(20000, 300, np.float64, 77)
+    bins = np.linspace(0.1, rmax, 5)
+    o = dict(periodic=True, boxsize=L, need_avg_sep=True)
+    kw = mode_kwargs("countpairs", X, bins=bins, L=L)
+    got = run(engine, "countpairs", options=_abi.make_options(**o), **kw)
+    want = run(oracle, "countpairs", "oracle_", options=_abi.make_options(**o), **kw)
+    assert_same("countpairs", got, want, what="rmax %g" % rmax)
