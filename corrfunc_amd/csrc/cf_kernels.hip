@@ -928,7 +928,10 @@ template __global__ void k_pairs_plain<true>(PairParams, DevLattice, DevLattice,
 // Either way every counted pair is decided by the reference's FP64 arithmetic.
 constexpr int kQueues = 8;          // work sub-queues (one counter each)
 constexpr int kCounterStride = 32;  // ints between sub-queue counters (128 B)
-constexpr int kFewGroups = 2;       // secondary windows up to this many groups are not box-tested
+// Secondary windows up to this many groups are not box-tested: the test's chain of
+// loads costs what the skipped groups save (uniform DD, kernel, with 2 / 4 / 8: 43
+// particles per cell 1.50 / 1.38 / 1.38 ms, 57 2.00 / 1.93 / 1.91, 115 5.32 / 5.32 / 5.49).
+constexpr int kFewGroups = 4;
 constexpr int kBlockJ = 4;          // secondaries per scalar load of the sparse path
 // Survivor buffer per wave: entries (j << 6) | lane at [head, tail). Drains take
 // 64 * DP entries from the head (DP survivors per lane: 1, or 2 with both pairs'

@@ -1,4 +1,4 @@
-"""Sparse grids, whose light cell pairs (at most 256 tests) are counted one lane per cell pair and
+"""Sparse grids, whose light cell pairs (at most 1024 tests) are counted one lane per cell pair and
 whose heavy ones by the persistent kernel: all modes against the oracle, with a clump that makes a
 few cell pairs heavy, at sizes around the limit, and batches with empty and one-point catalogs."""
 import os
@@ -22,7 +22,7 @@ def _sparse(n, clump, dtype, seed):
 
 
 @pytest.mark.parametrize("mode", MODES)
-@pytest.mark.parametrize("clump", [0, 15, 16, 17, 23, 200])
+@pytest.mark.parametrize("clump", [0, 15, 16, 17, 31, 32, 33, 46, 200])
 @pytest.mark.parametrize("avg", [False, True])
 def test_light_cell_pairs(engine, oracle, mode, clump, avg):
     os.environ["CORRFUNC_AMD_DENSE"] = "0"
