@@ -1479,7 +1479,8 @@ __device__ __forceinline__ void reg_groups(const PairParams& P, const CellPairRe
         const double dx = xj - xpos, dy = yj - ypos, dz = zj - zpos;
         double r2 = sep2<R2F>(dx, dy, dz);
         if (touch) {
-            const bool near = r2 >= P.near_lo2 && r2 < P.sqr_rmax;
+            // (a lane without a primary has a position, but no record i to replay)
+            const bool near = ivalid && r2 >= P.near_lo2 && r2 < P.sqr_rmax;
             if (__builtin_amdgcn_ballot_w64(near)) {
                 if (near) {
                     // the reference's pruning tests (see exact_pair)
