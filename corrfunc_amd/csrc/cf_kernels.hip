@@ -1471,7 +1471,9 @@ __device__ __forceinline__ void reg_groups(const PairParams& P, const CellPairRe
     unsigned cnt[NB];  // cumulative: pairs below e[b]
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        e[b] = b < NB - 1 || touch ? S.e[min(k0 + b, P.nbin - 1)] : DBL_MAX;
+        // (no edge above rmax: the last line of a bin file may end below an earlier one,
+        // and the differences of the cumulative counts need edges in order)
+        e[b] = b < NB - 1 || touch ? fmin(S.e[min(k0 + b, P.nbin - 1)], P.sqr_rmax) : DBL_MAX;
         if (!ivalid) e[b] = -1.0;  // no pair of a lane without a primary
         cnt[b] = 0;
     }

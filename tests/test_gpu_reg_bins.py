@@ -55,3 +55,39 @@ def test_lattice_in_a_captured_batch(engine, oracle):
                 assert_same("countpairs", got, want, what="graph")
     finally:
         g.close()
+
+
+def _edge_file(tmp_path, pairs):
+    f = tmp_path / "bins"
+    f.write_text("".join("%r %r\n" % p for p in pairs))
+    return str(f)
+
+
+@pytest.mark.parametrize("upper", [(5.0, 12.0, 9.0), (2.0, 12.0, 30.0, 9.0), (9.0, 9.0), (10.0, 9.0), (3.0, 6.0, 9.0)])
+@pytest.mark.parametrize("mode", MODES_1D)
+def test_last_edge_below_an_earlier_one(engine, oracle, tmp_path, mode, upper):
+    """rmax is the last line's upper edge, whichever edges lie above it: counts end there."""
+    rng = np.random.default_rng(len(upper))
+    X = [rng.uniform(0, 40.0, 40000) for _ in range(3)]
+    lower = (1.0,) + upper[:-1]
+    o = dict(periodic=True, boxsize=40.0, need_avg_sep=False)
+    kw = mode_kwargs(mode, X, bins=_edge_file(tmp_path, list(zip(lower, upper))), L=40.0, pimax=12.0)
+    got = run(engine, mode, options=_abi.make_options(**o), **kw)
+    want = run(oracle, mode, "oracle_", options=_abi.make_options(**o), **kw)
+    assert_same(mode, got, want, what="edges %s" % (upper,))
+
+
+def test_last_edge_below_an_earlier_one_in_a_captured_batch(engine, oracle, tmp_path):
+    rng = np.random.default_rng(9)
+    cats = [[rng.uniform(0, 40.0, 40000) for _ in range(3)] for _ in range(2)]
+    dev = [[_lib.DeviceArray(a) for a in x] for x in cats]
+    bins = _edge_file(tmp_path, [(1.0, 5.0), (5.0, 12.0), (12.0, 9.0)])
+    o = dict(periodic=True, boxsize=40.0, need_avg_sep=False)
+    g = _lib.BatchGraph([tuple(d) for d in dev], bins, options=_abi.make_options(**o))
+    try:
+        for x, got in zip(cats, g.launch()):
+            want = run(oracle, "countpairs", "oracle_", options=_abi.make_options(**o),
+                       **mode_kwargs("countpairs", x, bins=bins, L=40.0))
+            assert_same("countpairs", got, want, what="graph")
+    finally:
+        g.close()
