@@ -989,9 +989,16 @@ static const void* tuned_kernel(bool gh, int dp, int fl)
 }
 
 // Cell pairs of at most kLightPairs tests go to k_pairs_light when the cell pairs
-// have at most kLightMean tests on average (kernels, list alone and with the light
-// kernel: 78 tests 5.19 and 2.43 ms, 151 0.336 and 0.252, 255 0.337 and 0.415).
-constexpr int kLightPairs = 1024;
+// have at most kLightMean tests on average. The limit is on the one pair, since a
+// lane's tests are a serial chain (~0.25 us each): with 1024 a clustered catalog of
+// any size waits for its heaviest lanes. Kernels with all cell pairs in the list, and
+// with limits of 64 / 128 / 256 / 1024 tests, ms: 300 clustered points 0.060, 0.080 /
+// 0.102 / 0.152 / 0.245 (the light kernel saves the call 0.1 ms of host work); 16,000
+// 0.155, 0.179 / 0.201 / 0.253 / 0.387; uniform 100,000 points with 20 tests a cell
+// pair 0.67, 0.22 / 0.19 / 0.15 / 0.15, with 83 0.85, 0.68 / 0.38 / 0.31 / 0.33; 100
+// catalogs of 8,000 points with 105 5.34, 5.35 / 3.74 / 3.66 / 3.70. Beyond a mean of
+// about 160 the list has nearly all of the work.
+constexpr int kLightPairs = 128;
 constexpr double kLightMean = 160.0;
 constexpr size_t kLightLds = 40 * 1024;  // four workgroups of four waves per CU
 
@@ -1015,7 +1022,7 @@ static const void* light_kernel(const PairParams& P, int batch)
 // does not fit.
 static int launch_light(int ncp, const CellPairRec* cps, const DevLattice* lats, int batch, const PairParams& P0,
                         const double* d_edges, const unsigned short* d_lut, unsigned long long* g_np, double* g_avg,
-                        double* g_w, bool dry)
+                        double* g_w, int light, bool dry)
 {
     Engine& E = eng();
     PairParams P = P0;
@@ -1031,7 +1038,6 @@ static int launch_light(int ncp, const CellPairRec* cps, const DevLattice* lats,
     P.hist_copies = R;
     const long waves = (long)E.ncu * 16;
     // about four chunks a wave, in a batch long ones (a change of catalog flushes)
-    int light = kLightPairs;
     int chunk = (int)std::min<long>(batch ? 1024 : 256, std::max<long>(64, ((long)ncp / (4 * waves)) & ~63l));
     const long need = ((long)ncp + 4 * chunk - 1) / (4 * chunk);
     const unsigned blocks = (unsigned)std::max<long>(1, std::min<long>(need, waves / 4));
@@ -1218,9 +1224,13 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
     const int per_cu = ts.per_cu;
     const long max_blocks = (long)E.ncu * per_cu;
     // (per-cell-pair timings need every cell pair in the list)
-    const int light = !gh && !timed && !E.full_list && P.dense_mode == 0 && tested <= kLightMean * ncp &&
-                              launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, true)
-                          ? kLightPairs
+    // CORRFUNC_AMD_LIGHT: another limit (0: every cell pair in the list; for tests and sweeps)
+    const char* lp = getenv("CORRFUNC_AMD_LIGHT");
+    const int light_pairs = lp ? atoi(lp) : kLightPairs;
+    const int light = light_pairs > 0 && !gh && !timed && !E.full_list && P.dense_mode == 0 &&
+                              tested <= kLightMean * ncp &&
+                              launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, 0, true)
+                          ? light_pairs
                           : 0;
 
     // ---- cost prediction and order
@@ -1318,7 +1328,7 @@ static int launch_tuned(int ncp, const CellPairRec* cps, const DevLattice* lats,
 
     void* kargs[] = {&P, &lats, &cps, &items, &d_nitems, &counter, &d_edges, &d_lut, &g_np, &g_avg, &g_w, &ticks, &cu, &single};
     CF_CHECK(hipEventRecord(E.ev0, E.stream));
-    if (light) launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, false);
+    if (light) launch_light(ncp, cps, lats, batch, P, d_edges, d_lut, g_np, g_avg, g_w, light, false);
     if (!light || nitems > 0)
         CF_CHECK(hipLaunchKernel(kfn, dim3((unsigned)blocks), dim3(threads), kargs, lds, E.stream));
     CF_CHECK(hipGetLastError());
