@@ -436,6 +436,8 @@ static int make_grid(GridSpec& g, const double ext[6], const double gsz[3], cons
 // has an unclamped quantized offset.
 static double grid_qinv(const GridSpec& g) { return (double)kQMax / (fmax(g.xbs, fmax(g.ybs, g.zbs)) + g.qreach); }
 
+constexpr int64_t kCrowdedCell = 1024;  // particles a cell from which k_bucket_count_few takes a grid of few cells
+
 // Device counting sort of one particle set into the grid (gridlink_impl.c.src:65-436).
 // Counting-sort gridding launched on the stream without waiting: particles
 // outside the grid are counted into *oob (zeroed by the caller) and skipped.
@@ -474,7 +476,20 @@ static int gridlink_launch(const std::string& tag, const GridSpec& g, int64_t n,
     GridArgs ga{g.xmin, g.ymin, g.zmin, g.xinv, g.yinv, g.zinv, g.xbs, g.ybs, g.zbs, g.nx, g.ny, g.nz, L.qinv};
     const unsigned blocks = (unsigned)((n + 255) / 256);
     if (n > 0) {
-        if (esize == 4)
+        // few cells of a thousand particles and more: their atomics in LDS first (4M
+        // particles into 8 / 32 / 243 cells, to the end of gridding: 8.7 / 9.9 / 5.9 ms
+        // with k_bucket_count, 8.0 / 5.0 / 4.0 with k_bucket_count_few)
+        if (nb <= kFewCells && n >= nb * kCrowdedCell) {
+            const unsigned fb = (unsigned)((n + kFewItems - 1) / kFewItems);
+            if (esize == 4)
+                k_bucket_count_few<float><<<fb, 256, 0, E.stream>>>(n, (const float*)X, (const float*)Y,
+                                                                    (const float*)Z, ga, (int)nb, bucket, rank,
+                                                                    counts, oob);
+            else
+                k_bucket_count_few<double><<<fb, 256, 0, E.stream>>>(n, (const double*)X, (const double*)Y,
+                                                                     (const double*)Z, ga, (int)nb, bucket, rank,
+                                                                     counts, oob);
+        } else if (esize == 4)
             k_bucket_count<float><<<blocks, 256, 0, E.stream>>>(n, (const float*)X, (const float*)Y, (const float*)Z,
                                                                  ga, bucket, rank, counts, oob);
         else
