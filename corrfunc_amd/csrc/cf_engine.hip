@@ -1806,9 +1806,10 @@ static int run_core(const CallSpec& c, struct config_options* o, struct extra_op
 
 
 // ----------------------------------------------------------------- batches
-// DD(r) auto-correlations of many independent catalogs in one device work list
-// and one persistent pair-kernel launch. Catalog k gets exactly the results that
-// countpairs() gives for it with a copy of `options`.
+// Candidate cell pairs up to which a batch is gridded jointly (CORRFUNC_AMD_BATCH_CAND
+// lowers it): 256 catalogs of 50,000-2M points in 30 x 30 x 10 cells have 3.4e8.
+constexpr int64_t kJointCandidates = (int64_t)1 << 29;
+
 // Gridding and cell pairs of a whole batch in concatenated arrays (cf_batch.hip).
 // `sets` (ncat + 1 entries, inputs, extents' block numbers and grids filled in)
 // gets its offsets here; fills hl, the work list, its length and the pairs tested.
@@ -1917,6 +1918,9 @@ static int batch_grid(int ncat, std::vector<BatchSet>& sets, size_t esize, std::
     return EXIT_SUCCESS;
 }
 
+// DD(r) auto-correlations of many independent catalogs in one device work list
+// and one persistent pair-kernel launch. Catalog k gets exactly the results that
+// countpairs() gives for it with a copy of `options`.
 static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, void** W, const char* binfile,
                      struct config_options* options, struct extra_options* extra, std::vector<CallOut>& outs)
 {
@@ -1952,9 +1956,10 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
 
     // Phased over all catalogs, one host synchronisation per phase:
     //   1. inputs and extents            -> sync (extents)
-    //   2. grids (host), gridding        (no sync)
-    //   3. cell-pair flags + scans, counts gathered on the device -> sync
-    //   4. flags + scans again, records emitted into the concatenated list
+    //   2. grids (host), gridding, cell-pair flags and their scan -> sync (counts)
+    //   3. the records of the flagged candidates
+    // 2 and 3 are one launch a step over all catalogs (batch_grid); the largest
+    // batches take them catalog by catalog, and 3 then flags and scans again
     std::vector<DevLattice> hl(ncat);
     std::vector<const void*> dx(ncat), dy(ncat), dz(ncat), dw(ncat);
     for (int k = 0; k < ncat; k++) {
@@ -2051,9 +2056,9 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         for (int d = 0; d < 3; d++) rmaxr = refine[d] > rmaxr ? refine[d] : rmaxr;
     }
     coord_scale = 6 * coord_scale + wrap0[0] + wrap0[1] + wrap0[2] + rmax;
-    // all catalogs in concatenated arrays while these keep to 32-bit indices
-    // (96 catalogs of 2,000-20,000 points: 2,757 launches become 60), else one
-    // catalog after the other
+    // all catalogs in concatenated arrays while these keep to 32-bit indices and the
+    // candidates' flags and positions to 4 GiB (96 catalogs of 2,000-20,000 points: 2,757
+    // launches become 60), else one catalog after the other
     int64_t sum_n = 0, sum_cells = 0, sum_cand = 0;
     for (int k = 0; k < ncat; k++) {
         BatchSet& s = sets[k];
@@ -2068,7 +2073,9 @@ static int run_batch(int ncat, const int64_t* ND, void** X, void** Y, void** Z, 
         sum_cells += s.ncells;
         sum_cand += s.ncand;
     }
-    const bool joint = sum_n < (int64_t)INT32_MAX - 256 && sum_cells < (int64_t)INT32_MAX && sum_cand < (int64_t)1 << 30;
+    const char* jc = getenv("CORRFUNC_AMD_BATCH_CAND");
+    const int64_t max_cand = jc ? std::min<int64_t>(atoll(jc), kJointCandidates) : kJointCandidates;
+    const bool joint = sum_n < (int64_t)INT32_MAX - 256 && sum_cells < (int64_t)INT32_MAX && sum_cand <= max_cand;
     CellPairRec* cps = nullptr;
     int ncp_all = 0;
     if (joint) {
