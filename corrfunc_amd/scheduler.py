@@ -25,6 +25,7 @@ trained on per-cell-pair timings that the engine records itself:
 Counts are identical under every scheduler; only the kernel time changes.
 """
 import ctypes as C
+import warnings
 
 import numpy as np
 
@@ -127,12 +128,19 @@ def set_params(p, norm):
 
 def save(path):
     p, nm = params()
-    np.savez(path, params=p, norm=nm)
+    np.savez(path, params=p, norm=nm, features=np.array(FEATURE_NAMES))
 
 
 def load(path):
+    """Installs a saved model. One trained on other features than this engine computes (a file of an
+    earlier version does not name them) is installed with a warning: it predicts costs from values
+    it was not trained on, so it may order the work badly; counts do not depend on it."""
     with np.load(path, allow_pickle=False) as f:
+        names = tuple(str(n) for n in f["features"]) if "features" in f.files else None
         set_params(f["params"], f["norm"])
+    if names != FEATURE_NAMES:
+        warnings.warn("the cost model in %s was trained on other features than this engine computes; train it again"
+                      % path, RuntimeWarning, stacklevel=2)
 
 
 def predict(X):
