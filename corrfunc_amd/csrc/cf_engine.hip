@@ -934,9 +934,12 @@ static const DevLattice* lats_for(const DevLattice& L1, const DevLattice& L2)
 }
 
 // ---------------------------------------------------------- tuned launch
-// the queue hands out 4 items per atomic from 100 items per resident wave, when
-// there are at most 8 items per cell pair (few split cell pairs)
-constexpr int kBatchItemsPerWave = 100;
+// the queue hands out 4 items per atomic from 64 items per resident wave, when
+// there are at most 8 items per cell pair (few split cell pairs). Pair kernels with 1
+// and 4 items per atomic, ms: DDrppi, 547,000 items for 6,144 waves, 1.18 and 0.75;
+// DDsmu, 546,000, 1.17 and 0.73; DD, 776,000, 2.36 and 2.03; DDrppi, 307,000 for 4,096
+// waves, 2.18 and 2.04; with 8.5 items a wave equal (DDsmu, 52,000, 0.69 and 0.68)
+constexpr int kBatchItemsPerWave = 64;
 constexpr double kBatchItemsPerCellPair = 8.0;
 constexpr int kSplitPerWave = 4;  // a work item is split when it exceeds 1/(4 * resident waves) of the total cost
 
