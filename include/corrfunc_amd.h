@@ -33,7 +33,9 @@ typedef struct {
     int nmesh[3];            /* grid used by the last call */
     int refine[3];           /* bin refine factors used by the last call */
     int64_t num_cell_pairs;  /* neighbour-cell pairs in the work list */
-    int64_t num_work_items;  /* work items of the tuned kernel (0 for PLAIN) */
+    int64_t num_work_items;  /* work items of the tuned kernel (0 for PLAIN). On sparse grids (160 tests a
+                                cell pair and fewer on average) the cell pairs of at most 128 tests have
+                                none: one lane each counts them. 0 with cell pairs: all of them */
     double tested_pairs;     /* sum over cell pairs of N1*N2 (N(N-1)/2 for a cell with itself) */
     double kernel_ms;        /* pair-kernel time, HIP events on the engine's stream */
     double grid_ms;          /* host wall time from entry to the end of gridding */
