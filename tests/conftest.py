@@ -16,6 +16,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP engine)")
 
 
+@pytest.fixture(autouse=True)
+def engine_knobs_end_with_the_test():
+    """CORRFUNC_AMD_* variables that a test sets or removes are put back, whether it passes or fails."""
+    before = {k: v for k, v in os.environ.items() if k.startswith("CORRFUNC_AMD_")}
+    yield
+    for k in [k for k in os.environ if k.startswith("CORRFUNC_AMD_") and k not in before]:
+        del os.environ[k]
+    os.environ.update(before)
+
+
 @pytest.fixture(scope="session")
 def oracle():
     """The CPU oracle (FP64 restatement of the reference), bound with prefix oracle_."""
