@@ -2,7 +2,7 @@
 //
 // Device pipeline of one countpairs* call:
 //   k_minmax / k_minmax_final     data extent              (reference gridlink_utils.c.src:52-70)
-//   k_bucket_count                cell index per particle, cell histogram
+//   k_bucket_count (_few)         cell index per particle, cell histogram
 //                                                          (gridlink_impl.c.src:162-201)
 //   k_scan_*                      exclusive prefix sum of the cell histogram
 //   k_index_scatter               particle indices in cell order
