@@ -1010,12 +1010,12 @@ static const void* tuned_kernel(bool gh, int dp, int fl)
 // have at most kLightMean tests on average. The limit is on the one pair, since a
 // lane's tests are a serial chain (~0.25 us each): with 1024 a clustered catalog of
 // any size waits for its heaviest lanes. Kernels with all cell pairs in the list, and
-// with limits of 64 / 128 / 256 / 1024 tests, ms: 300 clustered points 0.060, 0.080 /
-// 0.102 / 0.152 / 0.245 (the light kernel saves the call 0.1 ms of host work); 16,000
-// 0.155, 0.179 / 0.201 / 0.253 / 0.387; uniform 100,000 points with 20 tests a cell
-// pair 0.67, 0.22 / 0.19 / 0.15 / 0.15, with 83 0.85, 0.68 / 0.38 / 0.31 / 0.33; 100
-// catalogs of 8,000 points with 105 5.34, 5.35 / 3.74 / 3.66 / 3.70. Beyond a mean of
-// about 160 the list has nearly all of the work.
+// with limits of 64 / 128 / 256 / 1024 tests, ms: 300 clustered points 0.059, 0.078 /
+// 0.103 / 0.154 / 0.249 (the light kernel saves the call 0.1 ms of host work); 16,000
+// 0.144, 0.187 / 0.206 / 0.258 / 0.390; uniform 100,000 points with 20 tests a cell
+// pair 0.69, 0.23 / 0.19 / 0.15 / 0.15, with 83 0.51, 0.73 / 0.38 / 0.31 / 0.33; 100
+// catalogs of 8,000 points with 105 5.46, 5.29 / 3.68 / 3.64 / 3.74. From a mean of
+// about 160 on most of the work is the list's.
 constexpr int kLightPairs = 128;
 constexpr double kLightMean = 160.0;
 constexpr size_t kLightLds = 40 * 1024;  // four workgroups of four waves per CU
